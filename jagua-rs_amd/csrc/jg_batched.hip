@@ -513,7 +513,87 @@ __global__ __launch_bounds__(WAVE, 4) void k_fused_filtered(const SetDesc* __res
     fused_loop<true, KIND>(sets, units, n_units, counters, m6, status, lds);
 }
 
+// One set without a table, for jg_detect_batch: the descriptor comes by value, workgroup b takes the
+// `chunk` queries from b * chunk on (then every gridDim.x-th unit), and runs both stages of them.
+// Nothing is allocated, claimed or left behind, so calls on any streams and threads, captured or
+// not, are independent.  A small batch is bound by the latency of one query's descent, so its
+// queries are spread over as many waves as the chip runs: 64 queries against a 40-item strip
+// take 18 us, 5000 against a 2000-item sheet 42 us; one query per lane, each descending by
+// itself, took 183 and 1227.
+template <bool FILT, int KIND>
+__global__ __launch_bounds__(WAVE, 4) void k_detect_direct(SetDesc sd, uint32_t n, uint32_t chunk,
+                                                           const float* __restrict__ m6, uint8_t* __restrict__ status) {
+    __shared__ WaveLds lds;
+    const WorkList W = wave_list(lds);
+    const uint32_t lane = threadIdx.x;
+    const uint32_t n_units = (n - 1u) / chunk + 1u;
+    for (uint32_t u = blockIdx.x; u < n_units; u += gridDim.x) {
+        const uint32_t q0 = u * chunk;
+        const Unit un{0u, q0, n - q0 < chunk ? n - q0 : chunk, 0u};
+        const uint64_t todo = surrogate_unit<FILT, KIND, FUSED_IPL>(sd, un, W, m6, status, lane);
+        if (todo != 0ull) poly_queries<FILT>(sd, q0, todo, W, m6, status, lane);
+        wave_sync();
+    }
+}
+
 // ---------------------------------------------------------------------------------------
+namespace {
+
+uint32_t device_cus() {
+    int dev = 0, cus = 256;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    return (uint32_t)cus;
+}
+
+}  // namespace
+
+namespace jg {
+
+bool detect_direct_fits(const jg_cde* c, uint64_t n) {
+    return c->view.n_nodes < WL_MAX_NODES && c->img.cap_edges <= WL_MAX_EDGES && n <= 0xffffffffull;
+}
+
+jg_status detect_direct_launch(const CdeView& cde, const ItemView& item, const FilterView& filter, uint32_t flags,
+                               const float* d_m6, uint64_t n, uint8_t* d_status, hipStream_t stream) {
+    SetDesc sd{};
+    sd.cde = cde;
+    sd.item = item;
+    sd.filter = filter;
+    sd.flags = flags;
+    // Queries per wave: one while the chip has waves to spare (16 per compute unit), then as few as
+    // keep the launch within that many, up to 16.  A wave's time grows with its queries long
+    // before its lanes are full, so small batches are quickest spread out; beyond 16 a unit's
+    // polygon stage is the tail.  Measured on a 2000-item layout (64-vertex item), us at 1 / 2 / 4 /
+    // 16 / 64 queries per wave: 1000 queries 28 / 29 / 32 / 41 / 115, 5000 44 / 42 / 43 / 55 / 137,
+    // 16384 70 / 52 / 45 / 56 / 135, 65536 211 / 130 / 89 / 72 / 146, 262144 781 / 452 / 282 / 179 / 189.
+    const uint64_t waves = (uint64_t)device_cus() * 16u;
+    uint32_t chunk = 1;
+    while (chunk < 16u && (n + chunk - 1) / chunk > waves) chunk <<= 1;
+    // lanes per query in the polygon stage: the plan's rule, and at least the wave over its queries
+    uint32_t lanes = 8;
+    while (lanes < item.n_v && lanes < 32u) lanes <<= 1;
+    sd.lanes = std::max(lanes, 64u / chunk);
+    const uint64_t units = (n + chunk - 1) / chunk;
+    const dim3 grid((uint32_t)std::min<uint64_t>(units, 1u << 20)), blk(WAVE);
+    const int kind = item.n_piers ? (item.n_poles ? KIND_MIXED : KIND_EDGE) : KIND_CIRCLE;
+#define JG_DIRECT(F, K) hipLaunchKernelGGL((k_detect_direct<F, K>), grid, blk, 0, stream, sd, (uint32_t)n, chunk, d_m6, d_status)
+#define JG_DIRECT_F(F)                                  \
+    if (kind == KIND_CIRCLE) JG_DIRECT(F, KIND_CIRCLE); \
+    else if (kind == KIND_EDGE) JG_DIRECT(F, KIND_EDGE); \
+    else JG_DIRECT(F, KIND_MIXED)
+    if (filter.kind != 0) {
+        JG_DIRECT_F(true);
+    } else {
+        JG_DIRECT_F(false);
+    }
+#undef JG_DIRECT_F
+#undef JG_DIRECT
+    return hip_check(hipGetLastError(), "detect launch");
+}
+
+}  // namespace jg
+
 namespace {
 
 
@@ -682,13 +762,6 @@ jg_status table_launch(const TableLayout& L, uint8_t* base, const float* d_m6, u
     }
 #undef JG_SURR
     return hip_check(hipGetLastError(), "batched query launch");
-}
-
-uint32_t device_cus() {
-    int dev = 0, cus = 256;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    return (uint32_t)cus;
 }
 
 }  // namespace

@@ -146,6 +146,13 @@ __device__ __forceinline__ bool pip_query_group(const ItemView& it, const Mat& m
     return (group_sum_i32(cnt, G) & 1) == 1;
 }
 
+// The batched detection's two stages over one set, described by value (jg_batched.hip): no table,
+// no allocation, one launch.  The traversal packs node numbers into 24 bits and hazard edges into
+// 29; detect_direct_fits says whether an engine and a batch are within them.
+bool detect_direct_fits(const jg_cde* c, uint64_t n);
+jg_status detect_direct_launch(const CdeView& cde, const ItemView& item, const FilterView& filter, uint32_t flags,
+                               const float* d_m6, uint64_t n, uint8_t* d_status, hipStream_t stream);
+
 // The batched hazard collection over a plan's table (jg_collect.hip): verdict-free, one set
 // per query.  ovf is a device list of n_queries (set, query) entries for the queries whose
 // sets outgrow the batched kernel's collector.
