@@ -291,8 +291,8 @@ JG_HD bool poly_has_point(const float2* v, uint32_t n, float4 bb, float x, float
     return (cnt & 1) == 1;
 }
 
-// Edge::distance_to(Point) (edge.rs:146-159, closest_point_on_edge :63-87)
-JG_HD float edge_point_dist(float4 e, float px, float py) {
+// Edge::distance_to(Point), squared (edge.rs:146-159, closest_point_on_edge :63-87)
+JG_HD float edge_point_sq_dist(float4 e, float px, float py) {
     const float a = px - e.x, b = py - e.y, c = e.z - e.x, d = e.w - e.y;
     const float dot = a * c + b * d;
     const float len_sq = c * c + d * d;
@@ -303,8 +303,9 @@ JG_HD float edge_point_dist(float4 e, float px, float py) {
     else if (param > 1.0f) { xx = e.z; yy = e.w; }
     else { xx = e.x + param * c; yy = e.y + param * d; }
     const float dx = px - xx, dy = py - yy;
-    return sqrtf(dx * dx + dy * dy);
+    return dx * dx + dy * dy;
 }
+JG_HD float edge_point_dist(float4 e, float px, float py) { return sqrtf(edge_point_sq_dist(e, px, py)); }
 
 // MAX_POI_TREE_DEPTH (fail_fast/pole.rs:82): levels below the root cell of the pole search
 constexpr int POLE_LEVELS = 10;
