@@ -137,6 +137,7 @@ static void set_view(jg_cde* c) {
     v.haz_verts = (const float2*)(b + im.o_vv);
     v.cells = (const uint32_t*)(b + im.o_ce);
     v.cell_level = im.cell_level;
+    v.grid = cell_grid(c->qt.pool[0].bbox, im.cell_level);
     v.n_slots = (uint32_t)im.slot_ver.size();
     v.exterior_slot = c->exterior.idx;
     v.cd_threshold = c->cfg.cd_threshold;

@@ -1,7 +1,8 @@
 // Batched persistent query form (jg_plan_*): many (engine, item, transform range) sets run
 // in one launch sequence fed by device work queues.
-//   k_surrogate: work units of up to 64 queries; lanes = (query, ff pole/pier) pairs, each
-//                lane descends from the root (cd_engine.rs:204-223).  Collisions are written
+//   k_surrogate: work units of up to 64 queries, first the cell of each query's first pole's
+//                centre, then the ff poles of the queries left from the cells that hold them and
+//                the piers from the root (cd_engine.rs:204-223).  Collisions are written
 //                out; the survivors of a unit are appended to the survivor queue in groups of
 //                one polygon-stage pass each (64/G queries, (set, first query, mask)).
 //   k_poly:      survivor groups; each query is handled by G lanes (G = the item's vertex
@@ -55,10 +56,14 @@ __device__ __forceinline__ WorkList wave_list(WaveLds& L) {
 constexpr int SURR_EG = 4;
 constexpr int POLY_EG = 1;
 
+// Units of more queries than this visit the cell of each query's first pole's centre by itself
+// first.  A few queries leave lanes idle either way, and then one traversal is the shorter chain.
+constexpr uint32_t CENTRE_MIN = 16;
+
 // The surrogate stage of one work unit (cd_engine.rs:204-223 for each of its queries): writes
 // the verdicts it settles and returns the mask of queries (bit i = query un.q0 + i) that go on
 // to the polygon stage.
-template <bool FILT, int KIND, int IPL>
+template <bool FILT, int KIND>
 __device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit& un, const WorkList& W,
                                                    const float* __restrict__ m6, uint8_t* __restrict__ status,
                                                    uint32_t lane) {
@@ -73,41 +78,82 @@ __device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit
     uint64_t hit_mask = 0;
     const uint32_t n_ent = (flags & JG_QUERY_SURROGATE) ? it.n_poles + it.n_piers : 0u;
     if (n_ent > 0) {
-        // every (query, ff pole / pier) of the unit descends from the root
-        // (cd_engine.rs:204-223), WL_ENT entities per traversal
+        const float4 root_bb = ldg_node(c.nodes).bbox;
         W.hit[lane] = 0u;
         if (FILT) W.qidx[lane] = un.q0 + lane;
-        const uint32_t total = cnt * n_ent;
-        for (uint32_t e0 = 0; e0 < total; e0 += WL_ENT) {
+        uint32_t first = 0u;                              // the node the first pass started from
+        // most queries collide where their first pole's centre lies: that one node per query first
+        const bool centre = KIND != KIND_EDGE && it.n_poles > 0u && cnt > CENTRE_MIN;
+        if (centre) {
             wave_sync();
-            uint32_t n = 0;
-            for (uint32_t j = 0; j < WL_ENT; j += WAVE) {
-                const uint32_t o = j + lane;
-                const uint32_t e = e0 + o;
-                bool want = false;
-                if (e < total) {
-                    const uint32_t qi = e / n_ent, k = e - qi * n_ent;
-                    if (!W.hit[qi]) {
-                        const Mat m = load_mat(m6, base + qi);
-                        const float4 p = ldg4(it.ff + k);
-                        const bool circle = k < it.n_poles;
-                        float4 gm;
-                        if (circle) {
-                            const float2 cc = xform(m, p.x, p.y);
-                            gm = make_float4(cc.x, cc.y, p.z, 0.0f);
-                        } else {
-                            const float2 a = xform(m, p.x, p.y), bb = xform(m, p.z, p.w);
-                            gm = make_float4(a.x, a.y, bb.x, bb.y);
-                        }
-                        W.geom[o] = gm;
-                        W.ent_slot[o] = (uint8_t)(qi | (circle ? WL_CIRCLE : 0u));
-                        want = true;
-                    }
-                }
-                n = wave_push_roots(W, n, want, o, 0u, lane);
+            if (lane < cnt) {
+                const Mat m = load_mat(m6, base + lane);
+                const float4 p = ldg4(it.ff);
+                const float2 cc = xform(m, p.x, p.y);
+                W.geom[lane] = make_float4(cc.x, cc.y, p.z, 0.0f);
+                W.ent_slot[lane] = (uint8_t)(lane | WL_CIRCLE);
+                first = centre_cell(c, root_bb, cc.x, cc.y);
             }
-            wave_traverse<FILT, KIND, IPL, SURR_EG>(c, f, W, n, lane);
+            const uint32_t n = wave_push_roots(W, 0u, lane < cnt, lane, first, lane);
+            wave_traverse<FILT, KIND, SURR_EG>(c, f, W, n, lane);
         }
+        // then every ff pole and pier of the queries not hit, pole by pole, up to WL_ENT entities per
+        // traversal (cd_engine.rs:204-223): a circle from the nodes of its cells, a pier from the root
+        uint32_t n = 0, n_e = 0;
+        wave_sync();
+        for (uint32_t k = 0; k < n_ent; k++) {
+            uint64_t live = __ballot(lane < cnt && W.hit[lane] == 0u);
+            if (live == 0ull) break;
+            const uint32_t add = (uint32_t)__builtin_popcountll(live);
+            if (n_e + add > WL_ENT || n + 4u * add > WL_NCAP - WL_RESERVE) {
+                wave_traverse<FILT, KIND, SURR_EG>(c, f, W, n, lane);
+                n = 0;
+                n_e = 0;
+                live = __ballot(lane < cnt && W.hit[lane] == 0u);
+                if (live == 0ull) break;
+            }
+            const bool want = (live >> lane) & 1ull;
+            const uint32_t o = n_e + lanes_below(live, lane);
+            uint32_t node[4], n_node = 0;
+            if (want) {
+                const Mat m = load_mat(m6, base + lane);
+                const float4 p = ldg4(it.ff + k);
+                const bool circle = k < it.n_poles;
+                float4 gm;
+                node[0] = 0u;
+                n_node = 1u;
+                if (circle) {
+                    const float2 cc = xform(m, p.x, p.y);
+                    gm = make_float4(cc.x, cc.y, p.z, 0.0f);
+                    const CircleCells cl = circle_cells(c.grid, c.cell_level, root_bb, cc.x, cc.y, p.z);
+                    const uint32_t* tab = c.cells + ((1u << (2u * cl.l)) - 1u) / 3u;
+                    const uint32_t a00 = ldg1(tab + ((cl.y0 << cl.l) | cl.x0)) & CELL_NODE;
+                    const uint32_t a01 = ldg1(tab + ((cl.y0 << cl.l) | cl.x1)) & CELL_NODE;
+                    const uint32_t a10 = ldg1(tab + ((cl.y1 << cl.l) | cl.x0)) & CELL_NODE;
+                    const uint32_t a11 = ldg1(tab + ((cl.y1 << cl.l) | cl.x1)) & CELL_NODE;
+                    const bool skip = centre && k == 0u;
+                    n_node = 0u;
+                    if (!(skip && a00 == first)) node[n_node++] = a00;
+                    if (a01 != a00 && !(skip && a01 == first)) node[n_node++] = a01;
+                    if (a10 != a00 && a10 != a01 && !(skip && a10 == first)) node[n_node++] = a10;
+                    if (a11 != a00 && a11 != a01 && a11 != a10 && !(skip && a11 == first)) node[n_node++] = a11;
+                } else {
+                    const float2 a = xform(m, p.x, p.y), bb = xform(m, p.z, p.w);
+                    gm = make_float4(a.x, a.y, bb.x, bb.y);
+                }
+                W.geom[o] = gm;
+                W.ent_slot[o] = (uint8_t)(lane | (circle ? WL_CIRCLE : 0u));
+            }
+            n_e += add;
+            const uint32_t incl = wave_incl_scan(n_node, lane);
+            const uint32_t at = n + incl - n_node;
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; j++)
+                if (j < n_node) W.nodes[at + j] = (o << 24) | node[j];
+            n += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        }
+        if (n != 0u) wave_traverse<FILT, KIND, SURR_EG>(c, f, W, n, lane);
+        wave_sync();
         hit_mask = __ballot(W.hit[lane] != 0u) & valid;
     }
     const uint64_t todo = (flags & JG_QUERY_POLY) ? (valid & ~hit_mask) : 0ull;
@@ -119,6 +165,12 @@ __device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit
     return todo;
 }
 
+// Bound by VALU issue of divergent lanes.  A descent from the root took about 8 levels of visits
+// for every pole; the cell tables give the nodes that can hold a pole's contacts at once
+// (circle_cells), and visiting the centre's cell by itself first leaves about a quarter of the
+// benchmark's queries for the rest.  1,048,576 queries over a 2000-item sheet: 337 -> 130 us
+// (without the centre's pass 300).  One item per lane and step: two measured 647 against 642 us
+// per step of both kernels once the descents were short.
 template <bool FILT, int KIND>
 __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict__ sets, const Unit* __restrict__ units,
                                                    uint32_t n_units, uint32_t* __restrict__ counters,
@@ -134,7 +186,7 @@ __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict
         const uint32_t u = claim_next(counters, C_USTREAM0, ux, utried, n_units, lane);
         if (u >= n_units) return;
         const Unit un = units[u];
-        const uint64_t todo = surrogate_unit<FILT, KIND, 2>(sets[un.set], un, W, m6, status, lane);
+        const uint64_t todo = surrogate_unit<FILT, KIND>(sets[un.set], un, W, m6, status, lane);
         if (todo != 0ull && lane == 0) {
             // one survivor group per polygon-stage pass (64 / G queries)
             const uint32_t per = 64u / sets[un.set].lanes;
@@ -376,7 +428,7 @@ __device__ __forceinline__ void poly_queries(const SetDesc& sd, uint32_t q0, uin
                 }
                 n = wave_push_roots(W, n, want, o, start, lane);
             }
-            wave_traverse<FILT, KIND_EDGE, 1, POLY_EG>(c, f, W, n, lane);
+            wave_traverse<FILT, KIND_EDGE, POLY_EG>(c, f, W, n, lane);
         }
         // containment over the virtual root's hazards (cd_engine.rs:176-193)
         wave_sync();
@@ -474,9 +526,6 @@ __global__ __launch_bounds__(WAVE, 5) void k_poly_filtered(const SetDesc* __rest
 // polygon stage of that unit's survivors itself.  No survivor queue is written, but the work of
 // a unit cannot spread: a unit of a large item with 30 survivors keeps one wave busy for about
 // 1.2 ms of a 1.34 ms configuration-2 step, so the two-kernel schedule is the default.
-// Items per lane of the fused kernel's surrogate stage.  2 fits in 90 VGPRs (4 waves per SIMD
-// kept) but measured 2% slower on the configuration-2 step than 1.
-constexpr int FUSED_IPL = 1;
 template <bool FILT, int KIND>
 __device__ __forceinline__ void fused_loop(const SetDesc* __restrict__ sets, const Unit* __restrict__ units,
                                            uint32_t n_units, uint32_t* __restrict__ counters,
@@ -490,7 +539,7 @@ __device__ __forceinline__ void fused_loop(const SetDesc* __restrict__ sets, con
         if (u >= n_units) break;
         const Unit un = units[u];
         const SetDesc& sd = sets[un.set];
-        const uint64_t todo = surrogate_unit<FILT, KIND, FUSED_IPL>(sd, un, W, m6, status, lane);
+        const uint64_t todo = surrogate_unit<FILT, KIND>(sd, un, W, m6, status, lane);
         if (todo != 0ull) poly_queries<FILT>(sd, un.q0, todo, W, m6, status, lane);
         wave_sync();
     }
@@ -530,7 +579,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_detect_direct(SetDesc sd, uint32_t 
     for (uint32_t u = blockIdx.x; u < n_units; u += gridDim.x) {
         const uint32_t q0 = u * chunk;
         const Unit un{0u, q0, n - q0 < chunk ? n - q0 : chunk, 0u};
-        const uint64_t todo = surrogate_unit<FILT, KIND, FUSED_IPL>(sd, un, W, m6, status, lane);
+        const uint64_t todo = surrogate_unit<FILT, KIND>(sd, un, W, m6, status, lane);
         if (todo != 0ull) poly_queries<FILT>(sd, q0, todo, W, m6, status, lane);
         wave_sync();
     }

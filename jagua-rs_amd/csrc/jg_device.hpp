@@ -91,7 +91,8 @@ struct CdeView {
     const uint32_t* cells;            // the deepest node on the path to each cell of a
                                       // 2^cell_level grid over the root box (row iy, column ix)
     uint32_t n_slots, exterior_slot, cd_threshold, n_nodes;
-    uint32_t cell_level, pad_[3];
+    uint32_t cell_level;
+    CellGrid grid;                    // the deepest table level's grid (circle_cells)
     float4 ext_inner;                 // a box inside the container (the exterior hazard's shape):
                                       // its bbox when that shape is an axis-aligned rectangle,
                                       // else empty (x_min > x_max)
@@ -282,6 +283,14 @@ __device__ __forceinline__ uint32_t start_node_below(const CdeView& c, uint32_t 
     }
     if (l == d0) return n0;
     return ldg1(c.cells + ((1u << (2u * l)) - 1u) / 3u + ((iy << l) | ix)) & CELL_NODE;
+}
+
+// The node of the deepest table level's cell that holds the circle's centre, or the nearest cell.
+__device__ __forceinline__ uint32_t centre_cell(const CdeView& c, float4 root, float cx, float cy) {
+    if (!(c.grid.sx > 0.0f)) return 0u;
+    const float top = (float)((1u << c.cell_level) - 1u);
+    const uint32_t ix = grid_index(cx - root.x, c.grid.sx, top), iy = grid_index(cy - root.y, c.grid.sy, top);
+    return ldg1(c.cells + ((1u << (2u * c.cell_level)) - 1u) / 3u + ((iy << c.cell_level) | ix)) & CELL_NODE;
 }
 
 // QTNode::collides for a circle (qt_node.rs:99-147; Circle quadrant test qt_traits.rs:10-13)
@@ -489,53 +498,40 @@ __device__ __forceinline__ uint32_t wave_push_roots(const WorkList& W, uint32_t 
 }
 
 // Runs the wave's nn pending node visits (and the edge tests they create) to completion;
-// W.hit[slot] is set for every query slot one of whose entities collides.  Callers push at
-// most WL_ENT roots (WL_ENT <= WL_NCAP).  Each lane handles IPL items per step (node visits or
-// edge tests): their memory reads are issued together, so a step waits for one round trip
-// instead of IPL.  An edge-test item holds up to EG consecutive edges of one hazard entry: a
-// leaf visit pushes one item per EG edges, so the lanes of a node step loop over a few pushes
-// each instead of one per edge (a leaf of the benchmark layout holds about 7 edges a circle
-// may meet), and an edge step tests up to EG edges per item.
-template <bool FILT, int KIND, int IPL = 1, int EG = 1>
+// W.hit[slot] is set for every query slot one of whose entities collides.  Callers push roots
+// into at most WL_NCAP - WL_RESERVE places.  An edge-test item holds up to EG consecutive edges
+// of one hazard entry: a leaf visit pushes one item per EG edges, so the lanes of a node step
+// loop over a few pushes each instead of one per edge (a leaf of the benchmark layout holds
+// about 7 edges a circle may meet), and an edge step tests up to EG edges per item.
+template <bool FILT, int KIND, int EG = 1>
 __device__ __forceinline__ void wave_traverse(const CdeView& c, const FilterView& f, const WorkList& W, uint32_t nn,
                                               uint32_t lane) {
-    static_assert(IPL == 1 || IPL == 2, "one or two items per lane");
     static_assert(EG >= 1 && EG <= 8, "one to eight edges per edge-test item");
-    // edge tests one item may push; the per-lane sum over IPL items stays below 2^16 / 64
-    constexpr uint32_t EDGE_LIMIT = IPL == 1 ? (1u << WL_EDGE_BITS) : (1u << (WL_EDGE_BITS - 1));
-    static_assert(64u * IPL * (EDGE_LIMIT - 1u) < 65536u, "a wave's edge pushes must fit 16 bits");
-    constexpr uint32_t STEP = 64u * IPL;
+    constexpr uint32_t EDGE_LIMIT = 1u << WL_EDGE_BITS;   // edge tests one visit may push: fewer
     uint32_t ne = 0;
     while (nn + ne != 0u) {
         wave_sync();                              // pushes and hit flags of the last step are visible
-        if (ne >= STEP || nn == 0u) {
-            // edge step: both tests' edges are read before either is evaluated
-            const uint32_t take = ne < STEP ? ne : STEP;
-            uint32_t eo[IPL], cnt[IPL];
-            float4 hedge[IPL][EG];
+        if (ne >= 64u || nn == 0u) {
+            // edge step: an item's edges are read before any is evaluated
+            const uint32_t take = ne < 64u ? ne : 64u;
+            const uint32_t at = lane < take ? ne - 1u - lane : 0u;
+            const uint32_t eo = W.edge_ent[at];
+            const uint32_t v = lane < take ? W.edges[at] : 0u;
+            const uint32_t e0 = v & WL_EDGE_INDEX, cnt = (v >> 29) + 1u;
+            float4 hedge[EG];
 #pragma unroll
-            for (int r = 0; r < IPL; r++) {
-                const uint32_t idx = lane + 64u * (uint32_t)r;
-                const uint32_t at = idx < take ? ne - 1u - idx : 0u;
-                eo[r] = W.edge_ent[at];
-                const uint32_t v = idx < take ? W.edges[at] : 0u;
-                const uint32_t e0 = v & WL_EDGE_INDEX;
-                cnt[r] = (v >> 29) + 1u;
-#pragma unroll
-                for (int k = 0; k < EG; k++) hedge[r][k] = ldg4(c.edges + e0 + ((uint32_t)k < cnt[r] ? (uint32_t)k : 0u));
-            }
-#pragma unroll
-            for (int r = 0; r < IPL; r++) {
-                if (lane + 64u * (uint32_t)r >= take) continue;
-                const uint32_t es = W.ent_slot[eo[r]];
+            for (int k = 0; k < EG; k++) hedge[k] = ldg4(c.edges + e0 + ((uint32_t)k < cnt ? (uint32_t)k : 0u));
+            if (lane < take) {
+                const uint32_t es = W.ent_slot[eo];
                 const uint32_t slot = es & 63u;
-                if (W.hit[slot]) continue;
-                const bool circle = KIND == KIND_CIRCLE || (KIND == KIND_MIXED && (es & WL_CIRCLE) != 0u);
-                const float4 gm = W.geom[eo[r]];
-                bool h = false;
+                if (!W.hit[slot]) {
+                    const bool circle = KIND == KIND_CIRCLE || (KIND == KIND_MIXED && (es & WL_CIRCLE) != 0u);
+                    const float4 gm = W.geom[eo];
+                    bool h = false;
 #pragma unroll
-                for (int k = 0; k < EG; k++) h = h || ((uint32_t)k < cnt[r] && edge_hit(circle, gm, hedge[r][k]));
-                if (h) W.hit[slot] = 1u;
+                    for (int k = 0; k < EG; k++) h = h || ((uint32_t)k < cnt && edge_hit(circle, gm, hedge[k]));
+                    if (h) W.hit[slot] = 1u;
+                }
             }
             ne -= take;
             continue;
@@ -548,146 +544,101 @@ __device__ __forceinline__ void wave_traverse(const CdeView& c, const FilterView
         uint32_t take = 1u;
         if (nn + 3u + WL_RESERVE <= WL_NCAP) {
             const uint32_t room = (WL_NCAP - WL_RESERVE - nn) / 3u;
-            take = nn < STEP ? nn : STEP;
+            take = nn < 64u ? nn : 64u;
             take = take < room ? take : room;
         }
         const uint32_t base = nn - take;
-        uint32_t item[IPL], m[IPL], n_edges[IPL], slot[IPL];
-        uint32_t p_beg[IPL], p_cnt[IPL], n_pass[IPL];   // a leaf's first passing entry's edges; passing entries
-                                                        // (kept with one item per lane)
-        int fc[IPL], s[IPL], he[IPL];
-        bool circle[IPL];
-        float4 g[IPL];
-        uint64_t q[IPL];
-        DevNode nd[IPL];
-#pragma unroll
-        for (int r = 0; r < IPL; r++) {                // the node records, all in flight together
-            const uint32_t idx = lane + 64u * (uint32_t)r;
-            item[r] = idx < take ? W.nodes[nn - 1u - idx] : 0u;
-            nd[r] = ldg_node(c.nodes + (item[r] & WL_NODE_MASK));
-        }
-        uint32_t packed = 0;
-#pragma unroll
-        for (int r = 0; r < IPL; r++) {
-            const uint32_t o = item[r] >> 24;
-            m[r] = 0;
-            n_edges[r] = 0;
-            if constexpr (IPL == 1) {
-                p_beg[r] = 0;
-                p_cnt[r] = 0;
-                n_pass[r] = 0;
-            }
-            fc[r] = 0;
-            s[r] = -1;
-            he[r] = 0;
-            slot[r] = 0;
-            circle[r] = KIND == KIND_CIRCLE;
-            g[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            q[r] = 0;
-            if (lane + 64u * (uint32_t)r < take) {
-                const uint32_t es = W.ent_slot[o];
-                slot[r] = es & 63u;
-                if (!W.hit[slot[r]]) {
-                    g[r] = W.geom[o];
-                    if (KIND == KIND_MIXED) circle[r] = (es & WL_CIRCLE) != 0u;
-                    if (FILT) q[r] = W.qidx[slot[r]];
-                    bool entire = false;
-                    s[r] = strongest_t<FILT>(c, nd[r], f, q[r], entire);
-                    if (s[r] >= 0 && entire) {
-                        W.hit[slot[r]] = 1u;
-                        s[r] = -1;
-                    } else if (s[r] >= 0 && nd[r].first_child >= 0) {
-                        fc[r] = nd[r].first_child;
-                        m[r] = circle[r] ? circle_quadrants(g[r].x, g[r].y, g[r].z, nd[r].bbox)
-                                         : edge_quadrants_node(g[r], nd[r].bbox);
-                        s[r] = -1;
-                    } else if (s[r] >= 0) {
-                        // leaf: count the edge tests of its relevant Partial hazards
-                        he[r] = (int)(nd[r].haz_begin + (nd[r].haz_info & COUNT_MASK));
-                        if constexpr (IPL == 1) {
-                            for (int i = s[r]; i < he[r]; i++) {
-                                const DevEntry e = ldg_ent(c.ent + i);
-                                if (!irrel<FILT>(f, q[r], e.slot_flags & SLOT_MASK) && ff_pass(e, circle[r], g[r])) {
-                                    if (n_pass[r] == 0u) {
-                                        p_beg[r] = e.edge_begin;
-                                        p_cnt[r] = e.edge_count;
-                                    }
-                                    n_pass[r]++;
-                                    n_edges[r] += (e.edge_count + (uint32_t)EG - 1u) / (uint32_t)EG;
-                                }
+        const uint32_t item = lane < take ? W.nodes[nn - 1u - lane] : 0u;
+        const uint32_t o = item >> 24;
+        const DevNode nd = ldg_node(c.nodes + (item & WL_NODE_MASK));
+        uint32_t m = 0, n_edges = 0, slot = 0;
+        uint32_t p_beg = 0, p_cnt = 0, n_pass = 0;    // a leaf's first passing entry's edges; passing entries
+        int fc = 0, s = -1, he = 0;
+        bool circle = KIND == KIND_CIRCLE;
+        float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        uint64_t q = 0;
+        if (lane < take) {
+            const uint32_t es = W.ent_slot[o];
+            slot = es & 63u;
+            if (!W.hit[slot]) {
+                g = W.geom[o];
+                if (KIND == KIND_MIXED) circle = (es & WL_CIRCLE) != 0u;
+                if (FILT) q = W.qidx[slot];
+                bool entire = false;
+                // a circle's start node is visited only if the circle meets its box (circle_cells);
+                // a pushed quadrant's box has passed the same test
+                if (KIND == KIND_EDGE || !circle || (item & WL_NODE_MASK) == 0u || circle_box(g.x, g.y, g.z, nd.bbox))
+                    s = strongest_t<FILT>(c, nd, f, q, entire);
+                if (s >= 0 && entire) {
+                    W.hit[slot] = 1u;
+                    s = -1;
+                } else if (s >= 0 && nd.first_child >= 0) {
+                    fc = nd.first_child;
+                    m = circle ? circle_quadrants(g.x, g.y, g.z, nd.bbox) : edge_quadrants_node(g, nd.bbox);
+                    s = -1;
+                } else if (s >= 0) {
+                    // leaf: count the edge tests of its relevant Partial hazards
+                    he = (int)(nd.haz_begin + (nd.haz_info & COUNT_MASK));
+                    for (int i = s; i < he; i++) {
+                        const DevEntry e = ldg_ent(c.ent + i);
+                        if (!irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g)) {
+                            if (n_pass == 0u) {
+                                p_beg = e.edge_begin;
+                                p_cnt = e.edge_count;
                             }
-                        } else {
-                            for (int i = s[r]; i < he[r]; i++) {
-                                const DevEntry e = ldg_ent(c.ent + i);
-                                if (!irrel<FILT>(f, q[r], e.slot_flags & SLOT_MASK) && ff_pass(e, circle[r], g[r]))
-                                    n_edges[r] += (e.edge_count + (uint32_t)EG - 1u) / (uint32_t)EG;
-                            }
+                            n_pass++;
+                            n_edges += (e.edge_count + (uint32_t)EG - 1u) / (uint32_t)EG;
                         }
                     }
                 }
             }
-            if (n_edges[r] >= EDGE_LIMIT) {
-                // more edge tests than one push carries: this lane tests the leaf's edges itself
-                bool h = false;
-                for (int i = s[r]; i < he[r] && !h; i++) {
-                    const DevEntry e = ldg_ent(c.ent + i);
-                    if (irrel<FILT>(f, q[r], e.slot_flags & SLOT_MASK) || !ff_pass(e, circle[r], g[r])) continue;
-                    for (uint32_t j = 0; j < e.edge_count && !h; j++) h = edge_hit(circle[r], g[r], ldg4(c.edges + e.edge_begin + j));
-                }
-                if (h) W.hit[slot[r]] = 1u;
-                n_edges[r] = 0;
-            }
-            // one scan for both pushes: child counts in the low 16 bits, edge counts in the high
-            // 16; neither sum over the wave carries out of its half
-            packed += (uint32_t)__builtin_popcount(m[r]) | (n_edges[r] << 16);
         }
+        auto test_leaf = [&]() {                      // this lane tests the leaf's edges itself
+            bool h = false;
+            for (int i = s; i < he && !h; i++) {
+                const DevEntry e = ldg_ent(c.ent + i);
+                if (irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) || !ff_pass(e, circle, g)) continue;
+                for (uint32_t j = 0; j < e.edge_count && !h; j++) h = edge_hit(circle, g, ldg4(c.edges + e.edge_begin + j));
+            }
+            if (h) W.hit[slot] = 1u;
+        };
+        if (n_edges >= EDGE_LIMIT) {                  // more edge tests than one push carries
+            test_leaf();
+            n_edges = 0;
+        }
+        // one scan for both pushes: child counts in the low 16 bits, edge counts in the high
+        // 16; neither sum over the wave carries out of its half
+        const uint32_t packed = (uint32_t)__builtin_popcount(m) | (n_edges << 16);
         const uint32_t incl = wave_incl_scan(packed, lane);
         const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         const uint32_t excl = incl - packed;
         const uint32_t n_tot = tot & 0xffffu, e_tot = tot >> 16;
-        wave_sync();                              // every lane has read its items before pushes overwrite
+        wave_sync();                              // every lane has read its item before pushes overwrite
         {
             uint32_t at = base + (excl & 0xffffu);     // base + n_tot <= WL_NCAP by the choice of take
-#pragma unroll
-            for (int r = 0; r < IPL; r++)
-                for (uint32_t b = m[r]; b; b &= b - 1u)
-                    W.nodes[at++] = (item[r] & ~WL_NODE_MASK) | (uint32_t)(fc[r] + __builtin_ctz(b));
+            for (uint32_t b = m; b; b &= b - 1u)
+                W.nodes[at++] = (item & ~WL_NODE_MASK) | (uint32_t)(fc + __builtin_ctz(b));
             nn = base + n_tot;
         }
         const bool fits = ne + e_tot <= WL_ECAP;
-        uint32_t at = ne + (excl >> 16);
-#pragma unroll
-        for (int r = 0; r < IPL; r++) {
-            if (!n_edges[r]) continue;
-            if (IPL == 1 && fits && n_pass[r] == 1u) {
-                // one passing entry (the common leaf): its edges from the count above (measured
-                // faster with one item per lane; with two, the extra registers cost more)
-                const uint32_t o = item[r] >> 24;
-                for (uint32_t j = 0; j < p_cnt[r]; j += EG, at++) {
-                    const uint32_t k = p_cnt[r] - j < (uint32_t)EG ? p_cnt[r] - j : (uint32_t)EG;
-                    W.edges[at] = (p_beg[r] + j) | ((k - 1u) << 29);
+        if (n_edges) {
+            uint32_t at = ne + (excl >> 16);
+            auto push = [&](uint32_t beg, uint32_t cnt) {
+                for (uint32_t j = 0; j < cnt; j += EG, at++) {
+                    const uint32_t k = cnt - j < (uint32_t)EG ? cnt - j : (uint32_t)EG;
+                    W.edges[at] = (beg + j) | ((k - 1u) << 29);
                     W.edge_ent[at] = (uint8_t)o;
                 }
-            } else if (fits) {
-                const uint32_t o = item[r] >> 24;
-                for (int i = s[r]; i < he[r]; i++) {
-                    const DevEntry e = ldg_ent(c.ent + i);
-                    if (irrel<FILT>(f, q[r], e.slot_flags & SLOT_MASK) || !ff_pass(e, circle[r], g[r])) continue;
-                    for (uint32_t j = 0; j < e.edge_count; j += EG, at++) {
-                        const uint32_t k = e.edge_count - j < (uint32_t)EG ? e.edge_count - j : (uint32_t)EG;
-                        W.edges[at] = (e.edge_begin + j) | ((k - 1u) << 29);
-                        W.edge_ent[at] = (uint8_t)o;
-                    }
-                }
+            };
+            if (!fits) {
+                test_leaf();                          // edge queue full
+            } else if (n_pass == 1u) {
+                push(p_beg, p_cnt);                   // one passing entry (the common leaf): its edges from the count above
             } else {
-                // edge queue full: this lane tests the leaf's edges itself
-                bool h = false;
-                for (int i = s[r]; i < he[r] && !h; i++) {
+                for (int i = s; i < he; i++) {
                     const DevEntry e = ldg_ent(c.ent + i);
-                    if (irrel<FILT>(f, q[r], e.slot_flags & SLOT_MASK) || !ff_pass(e, circle[r], g[r])) continue;
-                    for (uint32_t j = 0; j < e.edge_count && !h; j++) h = edge_hit(circle[r], g[r], ldg4(c.edges + e.edge_begin + j));
+                    if (!irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g)) push(e.edge_begin, e.edge_count);
                 }
-                if (h) W.hit[slot[r]] = 1u;
             }
         }
         if (fits) ne += e_tot;

@@ -249,6 +249,57 @@ JG_HD bool circle_box(float cx, float cy, float rad, float4 r) {
     float dx = nx - cx, dy = ny - cy;
     return dx * dx + dy * dy <= rad * rad;
 }
+// The even grid over a quadtree's root box at one level: cells per unit length (0: no usable
+// grid), and 2^-18 of the box's coordinates' magnitude.
+struct CellGrid {
+    float sx, sy, eps;
+};
+JG_HD CellGrid cell_grid(float4 root, uint32_t level) {
+    const float side = (float)(1u << level), sx = side / (root.z - root.x), sy = side / (root.w - root.y);
+    const float mag = mx(mx(fabsf(root.x), fabsf(root.z)), mx(fabsf(root.y), fabsf(root.w)));
+    const bool ok = level > 0u && sx > 0.0f && sy > 0.0f && sx <= 3.0e38f && sy <= 3.0e38f && mag <= 3.0e38f;
+    return CellGrid{ok ? sx : 0.0f, ok ? sy : 0.0f, ok ? mag * 0x1p-18f : 0.0f};
+}
+// The cell 0 .. top of an offset from the grid's lower bound; 0 for a NaN.
+JG_HD uint32_t grid_index(float off, float scale, float top) { return (uint32_t)mn(mx(off * scale, 0.0f), top); }
+
+// The start nodes of a circle's descent: the cells of one table level, at most 2 x 2, that hold the
+// circle, x0 .. x1 by y0 .. y1 of level l.
+//
+// The descent from the root ends, for a circle, in the nodes T that end it (a leaf, or one whose
+// strongest relevant hazard is Entire) with circle_box(T).  That test is hereditary in f32: the
+// distance per axis to a box inside another is no smaller, and subtraction, squares, the sum and
+// the comparison are monotone, so circle_box(T) holds for every node above T too, and the descent
+// reaches T (the argument of start_node_below covers the relevant hazards on the way).  A node's
+// box is met through its point nearest to the centre; the nodes below that hold this point have
+// the same nearest point, hence the same distance.  So it is enough to start at the nodes of
+// all cells that can hold such a point, each visited only if circle_box holds for it.  The point
+// is within the radius of the centre but for a few ulps, and a cell's bounds, midpoints of
+// midpoints, are a few ulps off the even grid: the interval is widened by 2^-18 of the radius and
+// of the root box's coordinates.  The root itself is visited without that test, as the search does.
+struct CircleCells {
+    uint32_t l, x0, x1, y0, y1;
+};
+JG_HD CircleCells circle_cells(const CellGrid& g, uint32_t level, float4 root, float cx, float cy, float r) {
+    CircleCells o{0u, 0u, 0u, 0u, 0u};
+    const float rp = r + r * 0x1p-18f + g.eps;
+    if (!(g.sx > 0.0f) || !(rp <= 3.0e38f)) return o;
+    const float top = (float)((1u << level) - 1u);
+    const uint32_t x0 = grid_index(cx - rp - root.x, g.sx, top);
+    const uint32_t x1 = grid_index(cx + rp - root.x, g.sx, top);
+    const uint32_t y0 = grid_index(cy - rp - root.y, g.sy, top);
+    const uint32_t y1 = grid_index(cy + rp - root.y, g.sy, top);
+    // the least shift that leaves at most two cells per axis
+    const uint32_t d = (x1 - x0 > y1 - y0 ? x1 - x0 : y1 - y0) >> 1;
+    uint32_t s = d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
+    if ((x1 >> s) - (x0 >> s) > 1u || (y1 >> s) - (y0 >> s) > 1u) s++;
+    o.l = level - s;
+    o.x0 = x0 >> s;
+    o.x1 = x1 >> s;
+    o.y0 = y0 >> s;
+    o.y1 = y1 >> s;
+    return o;
+}
 // circle.rs:109-113 via edge.rs:63-87,153-159  Circle–Edge
 JG_HD bool circle_edge(float cx, float cy, float rad, float4 e) {
     float a = cx - e.x, b = cy - e.y, c = e.z - e.x, d = e.w - e.y;
