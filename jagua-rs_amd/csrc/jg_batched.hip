@@ -33,21 +33,14 @@ using namespace jg;
 
 namespace {
 
-// LDS of a workgroup (one wavefront): its work list (within 8 KB, so that 20 waves share a CU)
-struct WaveLds {
-    uint32_t nodes[WL_NCAP];
-    uint32_t edges[WL_ECAP];
-    float4 geom[WL_ENT];
-    uint32_t hit[64];
-    uint32_t qidx[64];
-    uint8_t edge_ent[WL_ECAP];
-    uint8_t ent_slot[WL_ENT];
-};
+// LDS of a workgroup (one wavefront), for both stages and for the surrogate stage by itself, which
+// needs fewer entities and edge tests (563 -> 557 us per benchmark step).  The node queue must
+// have room to spare over the visits that are queued at once, as a step takes at most a third of
+// the room left: with 320 places a round of a local placement search, whose poles mostly miss,
+// took 214 us in k_surrogate instead of 57.
+using WaveLds = WorkList<512, 640, 128>;
+using SurrLds = WorkList<512, 320, 64>;
 static_assert(sizeof(WaveLds) <= 8192, "20 waves of a CU share its 160 KB of LDS");
-
-__device__ __forceinline__ WorkList wave_list(WaveLds& L) {
-    return WorkList{L.nodes, L.edges, L.edge_ent, L.geom, L.ent_slot, L.hit, L.qidx};
-}
 
 }  // namespace
 
@@ -63,8 +56,8 @@ constexpr uint32_t CENTRE_MIN = 16;
 // The surrogate stage of one work unit (cd_engine.rs:204-223 for each of its queries): writes
 // the verdicts it settles and returns the mask of queries (bit i = query un.q0 + i) that go on
 // to the polygon stage.
-template <bool FILT, int KIND>
-__device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit& un, const WorkList& W,
+template <bool FILT, int KIND, class Lds>
+__device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit& un, Lds& lds,
                                                    const float* __restrict__ m6, uint8_t* __restrict__ status,
                                                    uint32_t lane) {
     const CdeView c = sd.cde;
@@ -75,6 +68,8 @@ __device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit
     const uint32_t cnt = un.count;
     const uint64_t valid = cnt == 64 ? ~0ull : ((1ull << cnt) - 1ull);
 
+    using Traversal = WaveTraversal<FILT, KIND, SURR_EG, Lds>;
+    Lds& W = lds;
     uint64_t hit_mask = 0;
     const uint32_t n_ent = (flags & JG_QUERY_SURROGATE) ? it.n_poles + it.n_piers : 0u;
     if (n_ent > 0) {
@@ -82,78 +77,69 @@ __device__ __forceinline__ uint64_t surrogate_unit(const SetDesc& sd, const Unit
         W.hit[lane] = 0u;
         if (FILT) W.qidx[lane] = un.q0 + lane;
         uint32_t first = 0u;                              // the node the first pass started from
-        // most queries collide where their first pole's centre lies: that one node per query first
+        // most queries collide where their first pole's centre lies: that one node per query first.
+        // Then every ff pole and pier of the queries not hit, pole by pole, as many
+        // entities as the queue's room allows per traversal (cd_engine.rs:204-223): a circle from the
+        // nodes of its cells, a pier from the root.  (One loop, so that the traversal's code is there once.)
         const bool centre = KIND != KIND_EDGE && it.n_poles > 0u && cnt > CENTRE_MIN;
-        if (centre) {
+        Traversal T(c, f, W, lane);
+        bool at_centre = centre;
+        uint32_t k = 0;
+        for (;;) {
             wave_sync();
-            if (lane < cnt) {
-                const Mat m = load_mat(m6, base + lane);
-                const float4 p = ldg4(it.ff);
-                const float2 cc = xform(m, p.x, p.y);
-                W.geom[lane] = make_float4(cc.x, cc.y, p.z, 0.0f);
-                W.ent_slot[lane] = (uint8_t)(lane | WL_CIRCLE);
-                first = centre_cell(c, root_bb, cc.x, cc.y);
-            }
-            const uint32_t n = wave_push_roots(W, 0u, lane < cnt, lane, first, lane);
-            wave_traverse<FILT, KIND, SURR_EG>(c, f, W, n, lane);
-        }
-        // then every ff pole and pier of the queries not hit, pole by pole, up to WL_ENT entities per
-        // traversal (cd_engine.rs:204-223): a circle from the nodes of its cells, a pier from the root
-        uint32_t n = 0, n_e = 0;
-        wave_sync();
-        for (uint32_t k = 0; k < n_ent; k++) {
-            uint64_t live = __ballot(lane < cnt && W.hit[lane] == 0u);
-            if (live == 0ull) break;
-            const uint32_t add = (uint32_t)__builtin_popcountll(live);
-            if (n_e + add > WL_ENT || n + 4u * add > WL_NCAP - WL_RESERVE) {
-                wave_traverse<FILT, KIND, SURR_EG>(c, f, W, n, lane);
-                n = 0;
-                n_e = 0;
-                live = __ballot(lane < cnt && W.hit[lane] == 0u);
-                if (live == 0ull) break;
-            }
-            const bool want = (live >> lane) & 1ull;
-            const uint32_t o = n_e + lanes_below(live, lane);
-            uint32_t node[4], n_node = 0;
-            if (want) {
-                const Mat m = load_mat(m6, base + lane);
-                const float4 p = ldg4(it.ff + k);
-                const bool circle = k < it.n_poles;
-                float4 gm;
-                node[0] = 0u;
-                n_node = 1u;
-                if (circle) {
+            if (at_centre) {
+                float4 gm = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (lane < cnt) {
+                    const Mat m = load_mat(m6, base + lane);
+                    const float4 p = ldg4(it.ff);
                     const float2 cc = xform(m, p.x, p.y);
                     gm = make_float4(cc.x, cc.y, p.z, 0.0f);
-                    const CircleCells cl = circle_cells(c.grid, c.cell_level, root_bb, cc.x, cc.y, p.z);
-                    const uint32_t* tab = c.cells + ((1u << (2u * cl.l)) - 1u) / 3u;
-                    const uint32_t a00 = ldg1(tab + ((cl.y0 << cl.l) | cl.x0)) & CELL_NODE;
-                    const uint32_t a01 = ldg1(tab + ((cl.y0 << cl.l) | cl.x1)) & CELL_NODE;
-                    const uint32_t a10 = ldg1(tab + ((cl.y1 << cl.l) | cl.x0)) & CELL_NODE;
-                    const uint32_t a11 = ldg1(tab + ((cl.y1 << cl.l) | cl.x1)) & CELL_NODE;
-                    const bool skip = centre && k == 0u;
-                    n_node = 0u;
-                    if (!(skip && a00 == first)) node[n_node++] = a00;
-                    if (a01 != a00 && !(skip && a01 == first)) node[n_node++] = a01;
-                    if (a10 != a00 && a10 != a01 && !(skip && a10 == first)) node[n_node++] = a10;
-                    if (a11 != a00 && a11 != a01 && a11 != a10 && !(skip && a11 == first)) node[n_node++] = a11;
-                } else {
-                    const float2 a = xform(m, p.x, p.y), bb = xform(m, p.z, p.w);
-                    gm = make_float4(a.x, a.y, bb.x, bb.y);
+                    W.geom[lane] = gm;
+                    W.ent_slot[lane] = (uint8_t)(lane | WL_CIRCLE);
+                    first = centre_cell(c, root_bb, cc.x, cc.y);
                 }
-                W.geom[o] = gm;
-                W.ent_slot[o] = (uint8_t)(lane | (circle ? WL_CIRCLE : 0u));
-            }
-            n_e += add;
-            const uint32_t incl = wave_incl_scan(n_node, lane);
-            const uint32_t at = n + incl - n_node;
+                T.visit_start(lane < cnt, (lane << 24) | first, ldg_node(c.nodes + first), lane, true, gm);
+                at_centre = false;
+            } else {
+                const uint64_t live = __ballot(lane < cnt && W.hit[lane] == 0u);
+                const uint32_t add = (uint32_t)__builtin_popcountll(live);
+                if (live == 0ull || k == n_ent) break;
+                for (uint32_t n_e = 0; k < n_ent && n_e + add <= Traversal::ENT && T.nn + 4u * add <= Traversal::ROOT_ROOM; k++, n_e += add) {
+                    const bool want = (live >> lane) & 1ull;
+                    const uint32_t o = n_e + lanes_below(live, lane);
+                    uint32_t node[4] = {0u, 0u, 0u, 0u};
+                    bool start[4] = {want, false, false, false};
+                    if (want) {
+                        const Mat m = load_mat(m6, base + lane);
+                        const float4 p = ldg4(it.ff + k);
+                        const bool circle = k < it.n_poles;
+                        float4 gm;
+                        if (circle) {
+                            const float2 cc = xform(m, p.x, p.y);
+                            gm = make_float4(cc.x, cc.y, p.z, 0.0f);
+                            const CircleCells cl = circle_cells(c.grid, c.cell_level, root_bb, cc.x, cc.y, p.z);
+                            node[0] = cell_entry(c, cl.l, cl.x0, cl.y0) & CELL_NODE;
+                            node[1] = cell_entry(c, cl.l, cl.x1, cl.y0) & CELL_NODE;
+                            node[2] = cell_entry(c, cl.l, cl.x0, cl.y1) & CELL_NODE;
+                            node[3] = cell_entry(c, cl.l, cl.x1, cl.y1) & CELL_NODE;
+                            const bool skip = centre && k == 0u;         // visited by the centre's pass
+                            start[0] = !(skip && node[0] == first);
+                            start[1] = node[1] != node[0] && !(skip && node[1] == first);
+                            start[2] = node[2] != node[0] && node[2] != node[1] && !(skip && node[2] == first);
+                            start[3] = node[3] != node[0] && node[3] != node[1] && node[3] != node[2] && !(skip && node[3] == first);
+                        } else {
+                            const float2 a = xform(m, p.x, p.y), bb = xform(m, p.z, p.w);
+                            gm = make_float4(a.x, a.y, bb.x, bb.y);
+                        }
+                        W.geom[o] = gm;
+                        W.ent_slot[o] = (uint8_t)(lane | (circle ? WL_CIRCLE : 0u));
+                    }
 #pragma unroll
-            for (uint32_t j = 0; j < 4u; j++)
-                if (j < n_node) W.nodes[at + j] = (o << 24) | node[j];
-            n += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+                    for (uint32_t j = 0; j < 4u; j++) T.push_root(start[j], (o << 24) | node[j]);
+                }
+            }
+            T.run();
         }
-        if (n != 0u) wave_traverse<FILT, KIND, SURR_EG>(c, f, W, n, lane);
-        wave_sync();
         hit_mask = __ballot(W.hit[lane] != 0u) & valid;
     }
     const uint64_t todo = (flags & JG_QUERY_POLY) ? (valid & ~hit_mask) : 0ull;
@@ -177,8 +163,7 @@ __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict
                                                    Group* __restrict__ groups, const uint32_t* __restrict__ gbase,
                                                    const float* __restrict__ m6, uint8_t* __restrict__ status) {
     const uint32_t lane = threadIdx.x;
-    __shared__ WaveLds lds;
-    const WorkList W = wave_list(lds);
+    __shared__ SurrLds lds;
     // the polygon stage of this launch claims groups after this kernel: clear its claim counters
     if (blockIdx.x == 0 && lane < N_STREAMS) counters[C_STREAM0 + STREAM_STRIDE * lane] = 0u;
     uint32_t ux = blockIdx.x & (N_STREAMS - 1u), utried = 0;
@@ -186,7 +171,7 @@ __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict
         const uint32_t u = claim_next(counters, C_USTREAM0, ux, utried, n_units, lane);
         if (u >= n_units) return;
         const Unit un = units[u];
-        const uint64_t todo = surrogate_unit<FILT, KIND>(sets[un.set], un, W, m6, status, lane);
+        const uint64_t todo = surrogate_unit<FILT, KIND>(sets[un.set], un, lds, m6, status, lane);
         if (todo != 0ull && lane == 0) {
             // one survivor group per polygon-stage pass (64 / G queries)
             const uint32_t per = 64u / sets[un.set].lanes;
@@ -207,14 +192,14 @@ __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict
 }
 
 // detect_containment_collision (cd_engine.rs:231-255) over the candidates of one query, the
-// entries e0 .. e0 + cnt, by the query's G lanes (lane sub of the group starting at lane
-// base): true at the first that collides.  Each lane filters four candidates in flight (their
-// entries, then their bboxes and interior flags, read before any test): a shallow virtual root
-// holds up to every hazard of the layout.  A candidate without bbox relation collides iff its
-// scope is exterior; the point-in-polygon tests the filter leaves (hazard bbox surrounding, or
-// enclosed by, the query's) run on all G lanes, each polygon's edges split over them, since one
-// lane walking a container of thousands of vertices would hold the group.  The result is
-// containment()'s: interior ? contained : !contained, OR over the candidates.
+// entries e0 .. e0 + cnt, by G lanes (lane sub of the group starting at lane base): true at the
+// first that collides.  Each lane filters four candidates in flight (their entries, then their
+// bboxes and interior flags, read before any test): a shallow virtual root holds up to every
+// hazard of the layout.  A candidate without bbox relation collides iff its scope is exterior;
+// the point-in-polygon tests the filter leaves (hazard bbox surrounding, or enclosed by, the
+// query's) run on all G lanes, each polygon's edges split over them, since one lane walking a
+// container of thousands of vertices would hold the group.  The result is containment()'s:
+// interior ? contained : !contained, OR over the candidates.
 template <bool FILT>
 __device__ __forceinline__ bool scan_containment(const CdeView& c, const FilterView& f, uint64_t q, uint32_t e0,
                                                  uint32_t cnt, uint32_t sub, uint32_t G, uint32_t base,
@@ -236,15 +221,14 @@ __device__ __forceinline__ bool scan_containment(const CdeView& c, const FilterV
             iw[r] = ldg4(c.haz_poi + sl[r]).w;
         }
         bool direct = false;               // exterior scope, no bbox relation: !contained
-        uint32_t pend = 0;                 // bit r: candidate r needs its point-in-polygon test
-        int prel[CU];
+        uint32_t pend = 0, surr = 0;       // bit r: candidate r needs its point-in-polygon test; REL_SURROUNDING
 #pragma unroll
         for (uint32_t r = 0; r < CU; r++) {
-            prel[r] = REL_DISJOINT;
             if (k0 + r * G + sub >= cnt || irrel<FILT>(f, q, sl[r])) continue;
-            prel[r] = box_almost_relation(hb[r], bb);
-            if (prel[r] == REL_SURROUNDING || prel[r] == REL_ENCLOSED) pend |= 1u << r;
+            const int rel = box_almost_relation(hb[r], bb);
+            if (rel == REL_SURROUNDING || rel == REL_ENCLOSED) pend |= 1u << r;
             else if (iw[r] == 0.0f) direct = true;
+            if (rel == REL_SURROUNDING) surr |= 1u << r;
         }
         if ((ballot(direct) >> base) & gmask) return true;
 #pragma unroll
@@ -252,15 +236,11 @@ __device__ __forceinline__ bool scan_containment(const CdeView& c, const FilterV
             for (uint64_t pm = (ballot((pend >> r) & 1u) >> base) & gmask; pm; pm &= pm - 1ull) {
                 const int l = (int)base + __builtin_ctzll(pm);
                 const uint32_t s2 = (uint32_t)__shfl((int)sl[r], l, 64);
-                const int rl = __shfl(prel[r], l, 64);
-                bool contained;
-                if (rl == REL_SURROUNDING) {
-                    contained = pip_hazard_group(c, s2, qpoi.x, qpoi.y, sub, G);
-                } else {
-                    const float4 hp = ldg4(c.haz_poi + s2);
-                    contained = pip_query_group(it, m, bb, hp.x, hp.y, sub, G);
-                }
-                if (ldg4(c.haz_poi + s2).w != 0.0f ? contained : !contained) return true;
+                const bool rs = (__shfl((int)surr, l, 64) >> r) & 1;
+                const float4 hp = ldg4(c.haz_poi + s2);
+                const bool contained = rs ? pip_hazard_group(c, s2, qpoi.x, qpoi.y, sub, G)
+                                          : pip_query_group(it, m, bb, hp.x, hp.y, sub, G);
+                if (hp.w != 0.0f ? contained : !contained) return true;
             }
         }
     }
@@ -271,66 +251,10 @@ __device__ __forceinline__ bool scan_containment(const CdeView& c, const FilterV
 // the whole wave after the pass's other work, not by its own G lanes.
 constexpr uint32_t WAVE_SCAN_MIN = 64;
 
-// scan_containment for one query by the whole wave (all 64 lanes, the same arguments but
-// lane): candidates are filtered four per lane in flight; the point-in-polygon tests the
-// filter leaves (hazard bbox surrounding, or enclosed by, the query's) run on all 64 lanes,
-// since one lane walking a container of thousands of vertices would hold the wave.  The
-// result is the same: a candidate collides iff interior ? contained : !contained.
-template <bool FILT>
-__device__ __forceinline__ bool scan_containment_wave(const CdeView& c, const FilterView& f, uint64_t q, uint32_t e0,
-                                                      uint32_t cnt, uint32_t lane, const ItemView& it, const Mat& m,
-                                                      float4 bb, float2 qpoi) {
-    constexpr uint32_t CU = 4;
-    for (uint32_t k0 = 0; k0 < cnt; k0 += CU * 64u) {
-        uint32_t sl[CU];
-        float4 hb[CU];
-        float iw[CU];
-#pragma unroll
-        for (uint32_t r = 0; r < CU; r++) {
-            const uint32_t i = k0 + r * 64u + lane;
-            sl[r] = ldg_slot_flags(c.ent + e0 + (i < cnt ? i : 0u)) & SLOT_MASK;
-        }
-#pragma unroll
-        for (uint32_t r = 0; r < CU; r++) {
-            hb[r] = ldg4(c.haz_bbox + sl[r]);
-            iw[r] = ldg4(c.haz_poi + sl[r]).w;
-        }
-        bool direct = false;               // exterior scope, no bbox relation: !contained
-        uint32_t pend = 0;                 // bit r: candidate r needs its point-in-polygon test
-        int prel[CU];
-#pragma unroll
-        for (uint32_t r = 0; r < CU; r++) {
-            prel[r] = REL_DISJOINT;
-            if (k0 + r * 64u + lane >= cnt || irrel<FILT>(f, q, sl[r])) continue;
-            prel[r] = box_almost_relation(hb[r], bb);
-            if (prel[r] == REL_SURROUNDING || prel[r] == REL_ENCLOSED) pend |= 1u << r;
-            else if (iw[r] == 0.0f) direct = true;
-        }
-        if (ballot(direct) != 0ull) return true;
-#pragma unroll
-        for (uint32_t r = 0; r < CU; r++) {
-            for (uint64_t pm = ballot((pend >> r) & 1u); pm; pm &= pm - 1ull) {
-                const int l = __builtin_ctzll(pm);
-                const uint32_t s = (uint32_t)__shfl((int)sl[r], l, 64);
-                const int rl = __shfl(prel[r], l, 64);
-                bool contained;
-                if (rl == REL_SURROUNDING) {
-                    contained = pip_hazard_wave(c, s, qpoi.x, qpoi.y, lane);
-                } else {
-                    const float4 hp = ldg4(c.haz_poi + s);
-                    contained = pip_query_wave(it, m, bb, hp.x, hp.y, lane);
-                }
-                if (ldg4(c.haz_poi + s).w != 0.0f ? contained : !contained) return true;
-            }
-        }
-    }
-    return false;
-}
-
 // The polygon stage (cd_engine.rs:160-197) of the queries q0 + i for the set bits i of mask,
 // all of one set: 64/G queries per pass, G lanes each.
 template <bool FILT>
-__device__ __forceinline__ void poly_queries(const SetDesc& sd, uint32_t q0, uint64_t mask, const WorkList& W,
+__device__ __forceinline__ void poly_queries(const SetDesc& sd, uint32_t q0, uint64_t mask, WaveLds& W,
                                              const float* __restrict__ m6, uint8_t* __restrict__ status,
                                              uint32_t lane) {
     const CdeView c = sd.cde;
@@ -389,46 +313,52 @@ __device__ __forceinline__ void poly_queries(const SetDesc& sd, uint32_t q0, uin
         } else if (active) {
             vr = virtual_root_cells(c, root_bb, bb, vr_depth);
         }
-        // the virtual root's box and cell, below which the edges' start nodes are followed
-        float4 vbox = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        uint32_t vx = 0, vy = 0;
-        const bool vstart = active && vr_depth < c.cell_level;
-        if (vstart) {
-            vbox = ldg_node(c.nodes + vr).bbox;
-            node_cell(root_bb, vbox, vr_depth, vx, vy);
-        }
         // edges of the pass's unfinished queries, descending from their virtual roots
         // (cd_engine.rs:170-175), each from the deepest node below its virtual root known to
-        // hold it (start_node_below); a query slot is marked hit as soon as one edge collides
+        // hold it (edge_starts); a query slot is marked hit as soon as one edge collides
         wave_sync();
         if (sub == 0) {
             W.hit[slot] = done ? 1u : 0u;
             if (FILT) W.qidx[slot] = (uint32_t)q;
         }
-        // round R: lane (slot, sub) sets up edges sub + G (2R + j), j < WL_ENT / 64
-        constexpr uint32_t EPL = WL_ENT / WAVE;           // entities per lane per round
+        // round R: lane (slot, sub) sets up edges sub + G (2R + j), j < EPL, and makes their first visits
+        constexpr uint32_t EPL = WaveLds::ENT / WAVE;     // entities per lane per round
+        WaveTraversal<FILT, KIND_EDGE, POLY_EG, WaveLds> T(c, f, W, lane);
+        static_assert(2u * WaveLds::ENT <= decltype(T)::ROOT_ROOM, "two start nodes per entity");
         for (uint32_t i0 = 0; i0 < nv; i0 += EPL * G) {
             wave_sync();
-            if (__ballot(active && W.hit[slot] == 0u) == 0ull) break;
-            uint32_t n = 0;
+            const bool live = active && W.hit[slot] == 0u;
+            if (__ballot(live) == 0ull) break;
+            uint32_t n0[EPL], n1[EPL];
+            float4 gm[EPL];
+            DevNode nd[EPL];
+#pragma unroll
             for (uint32_t j = 0; j < EPL; j++) {
                 const uint32_t i = i0 + j * G + sub;
                 const uint32_t o = j * WAVE + lane;
-                const bool want = active && i < nv && W.hit[slot] == 0u;
-                uint32_t start = (uint32_t)vr;
-                if (want) {
+                n0[j] = n1[j] = (uint32_t)vr;
+                gm[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (live && i < nv) {
                     const uint32_t k = i + 1 == nv ? 0 : i + 1;
                     const float2 vi = ldg2(it.v + i), vk = ldg2(it.v + k);
                     const float2 a = xform(m, vi.x, vi.y);
                     const float2 b2 = xform(m, vk.x, vk.y);
-                    W.geom[o] = make_float4(a.x, a.y, b2.x, b2.y);
+                    gm[j] = make_float4(a.x, a.y, b2.x, b2.y);
+                    W.geom[o] = gm[j];
                     W.ent_slot[o] = (uint8_t)slot;
                     const float4 eb = make_float4(mn(a.x, b2.x), mn(a.y, b2.y), mx(a.x, b2.x), mx(a.y, b2.y));
-                    if (vstart) start = start_node_below(c, (uint32_t)vr, vr_depth, vbox, vx, vy, eb);
+                    edge_starts(c, root_bb, vr_depth, eb, n0[j], n1[j]);
                 }
-                n = wave_push_roots(W, n, want, o, start, lane);
             }
-            wave_traverse<FILT, KIND_EDGE, POLY_EG>(c, f, W, n, lane);
+#pragma unroll
+            for (uint32_t j = 0; j < EPL; j++) nd[j] = ldg_node(c.nodes + n0[j]);
+#pragma unroll
+            for (uint32_t j = 0; j < EPL; j++) {
+                const uint32_t o = (j * WAVE + lane) << 24;
+                T.push_root(n1[j] != n0[j], o | n1[j]);
+                T.visit_start(live && i0 + j * G + sub < nv, o | n0[j], nd[j], slot, false, gm[j]);
+            }
+            T.run();
         }
         // containment over the virtual root's hazards (cd_engine.rs:176-193)
         wave_sync();
@@ -467,7 +397,7 @@ __device__ __forceinline__ void poly_queries(const SetDesc& sd, uint32_t q0, uin
             const uint64_t qq = ((uint64_t)(uint32_t)__shfl((int)(uint32_t)(q >> 32), l0, 64) << 32) |
                                 (uint32_t)__shfl((int)(uint32_t)q, l0, 64);
             const float2 pq = xform(mq, it.poi.x, it.poi.y);
-            const bool any = scan_containment_wave<FILT>(c, f, qq, e0q, cq, lane, it, mq, bq, pq);
+            const bool any = scan_containment<FILT>(c, f, qq, e0q, cq, lane, 64u, 0u, it, mq, bq, pq);
             if ((int)(lane / G) == l0 / (int)G) hit = any;
         }
         const uint64_t bal = ballot(hit);
@@ -481,7 +411,6 @@ __device__ __forceinline__ void poly_loop(const SetDesc* __restrict__ sets, uint
                                           const Group* __restrict__ groups, const uint32_t* __restrict__ gbase,
                                           const float* __restrict__ m6, uint8_t* __restrict__ status, WaveLds& lds) {
     const uint32_t lane = threadIdx.x;
-    const WorkList W = wave_list(lds);
     // the surrogate stage of this launch is done: clear its unit-claim counters for the next
     if (blockIdx.x == 0 && lane < N_STREAMS) counters[C_USTREAM0 + STREAM_STRIDE * lane] = 0u;
     // stream x holds the groups its units appended; a wave drains its own stream, then the next
@@ -497,12 +426,19 @@ __device__ __forceinline__ void poly_loop(const SetDesc* __restrict__ sets, uint
             continue;
         }
         const Group gr = groups[gbase[x] + j];
-        poly_queries<FILT>(sets[gr.set], gr.q0, gr.mask, W, m6, status, lane);
+        poly_queries<FILT>(sets[gr.set], gr.q0, gr.mask, lds, m6, status, lane);
     }
     // every wave has read the group counts once the last one is out
     if (last_wave_out(counters, lane) && lane < N_STREAMS) counters[C_GCOUNT0 + STREAM_STRIDE * lane] = 0u;
 }
 
+// k_poly is bound by VALU issue (80% of SIMD cycles, half the lanes active), most of it the set-up and
+// the visits of the query edges.  On the 2000-item sheet, 1,048,576 queries: an edge's cell found by
+// one grid computation instead of a walk down the quadrants, and its first visit made from
+// registers, 643 -> 589 us per step of both kernels; two start nodes for an edge across one cell
+// side, which saves the descent from their common ancestor, 589 -> 564; unrolled containment
+// slots 564 -> 552.  A batch of 5000 queries of one item 37.7 -> 25.8 us.
+//
 // The two-stage kernels run 5 waves per SIMD (96 VGPRs, a few spilled; the LDS of a wave is
 // within 8 KB).  The filtered polygon stage carries the filter state on top and spills more at
 // 96, and still measured 4% faster on the filtered many-layout workload than at 4 waves; the
@@ -532,15 +468,14 @@ __device__ __forceinline__ void fused_loop(const SetDesc* __restrict__ sets, con
                                            const float* __restrict__ m6, uint8_t* __restrict__ status,
                                            WaveLds& lds) {
     const uint32_t lane = threadIdx.x;
-    const WorkList W = wave_list(lds);
     uint32_t ux = blockIdx.x & (N_STREAMS - 1u), utried = 0;
     for (;;) {
         const uint32_t u = claim_next(counters, C_USTREAM0, ux, utried, n_units, lane);
         if (u >= n_units) break;
         const Unit un = units[u];
         const SetDesc& sd = sets[un.set];
-        const uint64_t todo = surrogate_unit<FILT, KIND>(sd, un, W, m6, status, lane);
-        if (todo != 0ull) poly_queries<FILT>(sd, un.q0, todo, W, m6, status, lane);
+        const uint64_t todo = surrogate_unit<FILT, KIND>(sd, un, lds, m6, status, lane);
+        if (todo != 0ull) poly_queries<FILT>(sd, un.q0, todo, lds, m6, status, lane);
         wave_sync();
     }
     // every wave has stopped claiming once the last one is out
@@ -573,14 +508,13 @@ template <bool FILT, int KIND>
 __global__ __launch_bounds__(WAVE, 4) void k_detect_direct(SetDesc sd, uint32_t n, uint32_t chunk,
                                                            const float* __restrict__ m6, uint8_t* __restrict__ status) {
     __shared__ WaveLds lds;
-    const WorkList W = wave_list(lds);
     const uint32_t lane = threadIdx.x;
     const uint32_t n_units = (n - 1u) / chunk + 1u;
     for (uint32_t u = blockIdx.x; u < n_units; u += gridDim.x) {
         const uint32_t q0 = u * chunk;
         const Unit un{0u, q0, n - q0 < chunk ? n - q0 : chunk, 0u};
-        const uint64_t todo = surrogate_unit<FILT, KIND>(sd, un, W, m6, status, lane);
-        if (todo != 0ull) poly_queries<FILT>(sd, q0, todo, W, m6, status, lane);
+        const uint64_t todo = surrogate_unit<FILT, KIND>(sd, un, lds, m6, status, lane);
+        if (todo != 0ull) poly_queries<FILT>(sd, q0, todo, lds, m6, status, lane);
         wave_sync();
     }
 }

@@ -204,39 +204,6 @@ __device__ __forceinline__ int virtual_root(const CdeView& c, float4 bb) {
     return virtual_root(c, bb, depth);
 }
 
-// virtual_root through the cell tables: the quadrants of the root box (root: node 0's box) are
-// followed arithmetically (box_quadrant, the first quadrant that surrounds bb, as the search
-// takes it) down to the tables' deepest level or the first level where none surrounds bb; the
-// table entry of that cell is the deepest node on the path, where the search ends unless it
-// lies at the tables' deepest level, from which it goes on through node records.
-__device__ __forceinline__ int virtual_root_cells(const CdeView& c, float4 root, float4 bb, uint32_t& depth) {
-    int n = 0;
-    depth = 0;
-    if (c.cell_level > 0u) {
-        float4 r = root;
-        uint32_t ix = 0, iy = 0, l = 0;
-        for (; l < c.cell_level; l++) {
-            const int k = quadrant_surrounding(r, bb);
-            if (k < 0) break;
-            r = box_quadrant(r, k);
-            ix = 2u * ix + ((k == 0 || k == 3) ? 1u : 0u);
-            iy = 2u * iy + ((k == 0 || k == 1) ? 1u : 0u);
-        }
-        const uint32_t e = ldg1(c.cells + ((1u << (2u * l)) - 1u) / 3u + ((iy << l) | ix));
-        n = (int)(e & CELL_NODE);
-        depth = cell_depth(e);
-        if (depth < l || l < c.cell_level) return n;
-    }
-    for (;;) {
-        const DevNode nd = ldg_node(c.nodes + n);
-        if (nd.first_child < 0) return n;
-        const int k = quadrant_surrounding(nd.bbox, bb);
-        if (k < 0) return n;
-        n = nd.first_child + k;
-        depth++;
-    }
-}
-
 // The cell (ix, iy) at level `depth` of a node whose box `box` is a quadrant `depth` levels below
 // the root box: the quadrants holding the box's centre (strictly on one side of every midline
 // above it, as the box is one of the subdivision's).
@@ -254,35 +221,41 @@ __device__ __forceinline__ void node_cell(float4 root, float4 box, uint32_t dept
     }
 }
 
-// A node from which the descent of an edge with bounding box eb, starting at a node n0 that
-// holds it (depth d0 below the cell tables' deepest level, box box0, cell (x0, y0)), may start
-// instead: following the quadrant subdivision below n0 (box_quadrant's midpoints, the boxes the
-// tree's nodes have) while eb lies strictly inside one quadrant, down to the cell tables'
-// deepest level, the cell table gives the deepest node on that path (n0 when eb meets one of
-// n0's midlines).  No memory is read until that one entry.
-//
-// QTNode::collides from n0 visits this node with the same outcome.  Every hazard present below
-// a node is an entry of it (qt_node.rs:39-81: hazards reach children by constrict, and an
-// Entire hazard is Entire in every quadrant, qt_hazard.rs:58), and Entire entries come first
-// (qt_hazard_vec.rs), so along the path: an ancestor without relevant hazards leaves this node
-// none either, and an ancestor whose strongest relevant hazard is Entire leaves it Entire here
-// too.  An edge strictly inside each quadrant of the path collides with no quadrant off the
-// path at any ancestor (the box test of collides_with_quadrants finds those quadrants
-// disjoint, qt_traits.rs:19-106), so the ancestors' visits reduce to this one.
-__device__ __forceinline__ uint32_t start_node_below(const CdeView& c, uint32_t n0, uint32_t d0, float4 box0,
-                                                     uint32_t x0, uint32_t y0, float4 eb) {
-    float4 r = box0;
-    uint32_t ix = x0, iy = y0, l = d0;
-    for (; l < c.cell_level; l++) {
-        const float mxm = (r.x + r.z) / 2.0f, mym = (r.y + r.w) / 2.0f;
-        const bool xh = eb.x > mxm, xl = eb.z < mxm, yh = eb.y > mym, yl = eb.w < mym;
-        if (!(xh || xl) || !(yh || yl)) break;
-        r = make_float4(xh ? mxm : r.x, yh ? mym : r.y, xh ? r.z : mxm, yh ? r.w : mym);
-        ix = 2u * ix + (xh ? 1u : 0u);
-        iy = 2u * iy + (yh ? 1u : 0u);
+__device__ __forceinline__ uint32_t cell_entry(const CdeView& c, uint32_t l, uint32_t ix, uint32_t iy) {
+    return ldg1(c.cells + ((1u << (2u * l)) - 1u) / 3u + ((iy << l) | ix));
+}
+
+// virtual_root through the cell tables: at every level above the cell that strictly holds bb, that
+// cell's quadrant is the one that surrounds bb, so the search passes the deepest node on the path
+// to it; it ends there if that node lies above the cell's level, and goes on through node records
+// otherwise.  bb lies within the root box.
+__device__ __forceinline__ int virtual_root_cells(const CdeView& c, float4 root, float4 bb, uint32_t& depth) {
+    const HoldingCell h = holding_cell(c.grid, c.cell_level, root, bb);
+    const uint32_t e = cell_entry(c, h.l, h.ix, h.iy);
+    int n = (int)(e & CELL_NODE);
+    depth = cell_depth(e);
+    if (depth < h.l) return n;
+    for (;;) {
+        const DevNode nd = ldg_node(c.nodes + n);
+        if (nd.first_child < 0) return n;
+        const int k = quadrant_surrounding(nd.bbox, bb);
+        if (k < 0) return n;
+        n = nd.first_child + k;
+        depth++;
     }
-    if (l == d0) return n0;
-    return ldg1(c.cells + ((1u << (2u * l)) - 1u) / 3u + ((iy << l) | ix)) & CELL_NODE;
+}
+
+// The nodes from which the descent of an edge with bounding box eb, starting at a node n0 of depth
+// d0 that holds it, may start instead: the deepest nodes on the paths to its cells (edge_cells),
+// one or two of them (n1 = n0 then), when the cells lie below n0.
+__device__ __forceinline__ void edge_starts(const CdeView& c, float4 root, uint32_t d0, float4 eb, uint32_t& n0, uint32_t& n1) {
+    const EdgeCells e = edge_cells(c.grid, c.cell_level, root, eb);
+    if (e.l > d0) {
+        n0 = cell_entry(c, e.l, e.x0, e.y0) & CELL_NODE;
+        n1 = e.x0 != e.x1 || e.y0 != e.y1 ? cell_entry(c, e.l, e.x1, e.y1) & CELL_NODE : n0;
+    } else {
+        n1 = n0;
+    }
 }
 
 // The node of the deepest table level's cell that holds the circle's centre, or the nearest cell.
@@ -364,13 +337,9 @@ __device__ __forceinline__ bool collides_edge(const CdeView& c, int start, float
 // KIND_MIXED reads the per-entity kind (surrogates with both poles and piers).
 enum : int { KIND_EDGE = 0, KIND_CIRCLE = 1, KIND_MIXED = 2 };
 
-constexpr uint32_t WL_ENT = 128;          // entities per traversal
-constexpr uint32_t WL_NCAP = 512;         // node-visit queue entries per wave
-constexpr uint32_t WL_ECAP = 640;         // edge-test queue entries per wave (LDS within 8 KB: 20 waves per CU)
 constexpr int WL_EDGE_BITS = 10;          // edge tests one leaf visit pushes: fewer than 2^WL_EDGE_BITS
 static_assert(64u * ((1u << WL_EDGE_BITS) - 1u) < 65536u, "a wave's edge pushes must fit 16 bits");
 constexpr uint32_t WL_RESERVE = 3u * (JG_MAX_QT_DEPTH + 1u);   // node slots a depth-first walk may need
-static_assert(WL_NCAP >= WL_ENT + WL_RESERVE + 3u, "node queue must hold the roots and the reserve");
 constexpr uint32_t WL_NODE_MASK = 0xffffffu;
 constexpr uint32_t WL_MAX_NODES = 1u << 24;
 constexpr uint32_t WL_CIRCLE = 0x80u;     // WorkList::ent_slot flag: the entity is a circle
@@ -379,14 +348,17 @@ constexpr uint32_t WL_CIRCLE = 0x80u;     // WorkList::ent_slot flag: the entity
 constexpr uint32_t WL_EDGE_INDEX = 0x1fffffffu;
 constexpr uint32_t WL_MAX_EDGES = WL_EDGE_INDEX + 1u;
 
-struct WorkList {                         // per-wave LDS
-    uint32_t* nodes;                      // [WL_NCAP] entity << 24 | node
-    uint32_t* edges;                      // [WL_ECAP] hazard edges (WL_EDGE_INDEX)
-    uint8_t* edge_ent;                    // [WL_ECAP] entity of the edge test
-    float4* geom;                         // [WL_ENT] circle (cx, cy, r, -) or edge (x1 y1 x2 y2)
-    uint8_t* ent_slot;                    // [WL_ENT] query slot (0..63) | WL_CIRCLE
-    uint32_t* hit;                        // [64] per query slot
-    uint32_t* qidx;                       // [64] per query slot: query index (hashed filters)
+// A wave's work list in LDS: NCAP_ node visits, ECAP_ edge tests, ENT_ entities.
+template <uint32_t NCAP_, uint32_t ECAP_, uint32_t ENT_>
+struct WorkList {
+    static constexpr uint32_t NCAP = NCAP_, ECAP = ECAP_, ENT = ENT_;
+    uint32_t nodes[NCAP];                 // entity << 24 | node
+    uint32_t edges[ECAP];                 // hazard edges (WL_EDGE_INDEX)
+    float4 geom[ENT];                     // circle (cx, cy, r, -) or edge (x1 y1 x2 y2)
+    uint32_t hit[64];                     // per query slot
+    uint32_t qidx[64];                    // per query slot: query index (hashed filters)
+    uint8_t edge_ent[ECAP];               // entity of the edge test
+    uint8_t ent_slot[ENT];                // query slot (0..63) | WL_CIRCLE
 };
 
 template <bool FILT>
@@ -413,58 +385,12 @@ __device__ __forceinline__ bool edge_hit(bool circle, float4 g, float4 he) {
     return circle ? circle_edge(g.x, g.y, g.z, he) : edge_edge(g, he);
 }
 
-// QTHazPartial::collides_with over the relevant Partial entries of a leaf, from entry s on
-// (qt_node.rs:126-141, qt_partial_hazard.rs:67-72).
-template <bool FILT>
-__device__ __forceinline__ bool leaf_hits(const CdeView& c, const DevNode& nd, int s, bool circle, float4 g,
-                                          const FilterView& f, uint64_t q) {
-    const int he = (int)(nd.haz_begin + (nd.haz_info & COUNT_MASK));
-    for (int i = s; i < he; i++) {
-        const DevEntry e = c.ent[i];
-        if (irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) || !ff_pass(e, circle, g)) continue;
-        for (uint32_t j = 0; j < e.edge_count; j++)
-            if (edge_hit(circle, g, c.edges[e.edge_begin + j])) return true;
-    }
-    return false;
-}
-
-// One visit of QTNode::collides: HIT, or the mask of children to visit (first child in fc).
-template <bool FILT>
-__device__ __forceinline__ uint32_t visit_node(const CdeView& c, int n, bool circle, float4 g, const FilterView& f,
-                                               uint64_t q, int& fc) {
-    const DevNode nd = c.nodes[n];
-    bool entire = false;
-    const int s = strongest_t<FILT>(c, nd, f, q, entire);
-    if (s < 0) return 0u;
-    if (entire) return HIT;
-    if (nd.first_child >= 0) {
-        fc = nd.first_child;
-        if (circle) return circle_quadrants(g.x, g.y, g.z, nd.bbox);
-        return edge_quadrants_node(g, nd.bbox);
-    }
-    return leaf_hits<FILT>(c, nd, s, circle, g, f, q) ? HIT : 0u;
-}
-
 // The workgroup is a single wavefront: a convergent barrier ordering its lanes' LDS accesses.
 __device__ __forceinline__ void wave_sync() { __syncthreads(); }
 
 // Number of set bits of m below this lane.
 __device__ __forceinline__ uint32_t lanes_below(uint64_t m, uint32_t lane) {
     return (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull));
-}
-
-// Exclusive prefix sum over the wave of per-lane counts x < 2^BITS, one ballot per bit;
-// total (the sum) is wave-uniform.
-template <int BITS>
-__device__ __forceinline__ uint32_t wave_prefix(uint32_t x, uint32_t lane, uint32_t& total) {
-    uint32_t off = 0, tot = 0;
-    for (int b = 0; b < BITS; b++) {
-        const uint64_t bb = __ballot((x >> b) & 1u);
-        off += lanes_below(bb, lane) << b;
-        tot += (uint32_t)__builtin_popcountll(bb) << b;
-    }
-    total = tot;
-    return off;
 }
 
 // Inclusive prefix sum of x over the 64 lanes of a wave with every lane active: DPP row shifts
@@ -487,164 +413,230 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, uint32_t lane) {
     return v;
 }
 
-// Pushes one node visit per lane with want set onto a node queue of depth n (callers set
-// geom/ent_slot first); returns the new depth, the same in every lane.
-__device__ __forceinline__ uint32_t wave_push_roots(const WorkList& W, uint32_t n, bool want, uint32_t ent,
-                                                    uint32_t node, uint32_t lane) {
-    uint32_t total;
-    const uint32_t off = wave_prefix<1>(want ? 1u : 0u, lane, total);
-    if (want) W.nodes[n + off] = (ent << 24) | node;
-    return n + total;
-}
-
-// Runs the wave's nn pending node visits (and the edge tests they create) to completion;
-// W.hit[slot] is set for every query slot one of whose entities collides.  Callers push roots
-// into at most WL_NCAP - WL_RESERVE places.  An edge-test item holds up to EG consecutive edges
-// of one hazard entry: a leaf visit pushes one item per EG edges, so the lanes of a node step
-// loop over a few pushes each instead of one per edge (a leaf of the benchmark layout holds
-// about 7 edges a circle may meet), and an edge step tests up to EG edges per item.
-template <bool FILT, int KIND, int EG = 1>
-__device__ __forceinline__ void wave_traverse(const CdeView& c, const FilterView& f, const WorkList& W, uint32_t nn,
-                                              uint32_t lane) {
+// The node visits and edge tests of a wave's entities.  W.hit[slot] is set for every query slot one
+// of whose entities collides.  Callers queue visits with push_root or make an entity's first from
+// registers (visit_start); run() works the queues off.
+// An edge-test item holds up to EG consecutive edges of one hazard entry: a leaf visit pushes one
+// item per EG edges, so the lanes of a node step loop over a few pushes each instead of one per
+// edge (a leaf of the benchmark layout holds about 7 edges a circle may meet), and an edge step
+// tests up to EG edges per item.
+//
+// A round's chain of dependent reads is what a small launch waits for, and the steps' instructions on
+// half-empty waves what a large one does; a first visit from registers saves a step of both, and an
+// internal start node is left to run(), whose code is there once (in copies per set-up: 591 us per
+// benchmark step against 564).
+template <bool FILT, int KIND, int EG, class Lds>
+struct WaveTraversal {
     static_assert(EG >= 1 && EG <= 8, "one to eight edges per edge-test item");
-    constexpr uint32_t EDGE_LIMIT = 1u << WL_EDGE_BITS;   // edge tests one visit may push: fewer
-    uint32_t ne = 0;
-    while (nn + ne != 0u) {
-        wave_sync();                              // pushes and hit flags of the last step are visible
-        if (ne >= 64u || nn == 0u) {
-            // edge step: an item's edges are read before any is evaluated
-            const uint32_t take = ne < 64u ? ne : 64u;
-            const uint32_t at = lane < take ? ne - 1u - lane : 0u;
-            const uint32_t eo = W.edge_ent[at];
-            const uint32_t v = lane < take ? W.edges[at] : 0u;
-            const uint32_t e0 = v & WL_EDGE_INDEX, cnt = (v >> 29) + 1u;
-            float4 hedge[EG];
-#pragma unroll
-            for (int k = 0; k < EG; k++) hedge[k] = ldg4(c.edges + e0 + ((uint32_t)k < cnt ? (uint32_t)k : 0u));
-            if (lane < take) {
-                const uint32_t es = W.ent_slot[eo];
-                const uint32_t slot = es & 63u;
-                if (!W.hit[slot]) {
-                    const bool circle = KIND == KIND_CIRCLE || (KIND == KIND_MIXED && (es & WL_CIRCLE) != 0u);
-                    const float4 gm = W.geom[eo];
-                    bool h = false;
-#pragma unroll
-                    for (int k = 0; k < EG; k++) h = h || ((uint32_t)k < cnt && edge_hit(circle, gm, hedge[k]));
-                    if (h) W.hit[slot] = 1u;
-                }
-            }
-            ne -= take;
-            continue;
-        }
-        // node step.  An item pushes at most 4 children, 3 more slots than it frees, so taking t
-        // items grows the queue by at most 3t: steps take no more than keeps WL_RESERVE slots
-        // free.  Within the reserve, single-item steps walk depth-first, which grows the queue by
-        // at most 3 per level below where the walk began; the reserve covers the deepest tree.
-        // The queue therefore never overflows and every step makes progress.
-        uint32_t take = 1u;
-        if (nn + 3u + WL_RESERVE <= WL_NCAP) {
-            const uint32_t room = (WL_NCAP - WL_RESERVE - nn) / 3u;
-            take = nn < 64u ? nn : 64u;
-            take = take < room ? take : room;
-        }
-        const uint32_t base = nn - take;
-        const uint32_t item = lane < take ? W.nodes[nn - 1u - lane] : 0u;
-        const uint32_t o = item >> 24;
-        const DevNode nd = ldg_node(c.nodes + (item & WL_NODE_MASK));
-        uint32_t m = 0, n_edges = 0, slot = 0;
-        uint32_t p_beg = 0, p_cnt = 0, n_pass = 0;    // a leaf's first passing entry's edges; passing entries
-        int fc = 0, s = -1, he = 0;
-        bool circle = KIND == KIND_CIRCLE;
-        float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    static constexpr uint32_t NCAP = Lds::NCAP, ECAP = Lds::ECAP, ENT = Lds::ENT;
+    static constexpr uint32_t EDGE_LIMIT = 1u << WL_EDGE_BITS;   // edge tests one visit may push: fewer
+    static constexpr uint32_t ROOT_ROOM = NCAP - WL_RESERVE - 3u;   // node visits that callers may queue
+
+    const CdeView& c;
+    const FilterView& f;
+    Lds& W;
+    const uint32_t lane;
+    uint32_t nn = 0, ne = 0;                      // queued node visits and edge tests
+
+    __device__ __forceinline__ WaveTraversal(const CdeView& c_, const FilterView& f_, Lds& W_, uint32_t lane_)
+        : c(c_), f(f_), W(W_), lane(lane_) {}
+
+    // Queues one visit (entity << 24 | node) per lane with `want` set; callers keep nn within
+    // ROOT_ROOM.
+    __device__ __forceinline__ void push_root(bool want, uint32_t item) {
+        const uint64_t b = __ballot(want);
+        if (want) W.nodes[nn + lanes_below(b, lane)] = item;
+        nn += (uint32_t)__builtin_popcountll(b);
+    }
+
+    // The entities' first visits, one per lane with `act` set, from registers: the start node's record
+    // nd, the entity's query slot, kind and geometry (also in W.geom).  Most start nodes are leaves, and
+    // most of those empty; a leaf's edge tests are queued, and what is more than that (an internal
+    // node, more edges than the queue takes) queues the visit itself for run().
+    __device__ __forceinline__ void visit_start(bool act, uint32_t item, const DevNode& nd, uint32_t slot, bool circle, float4 g) {
+        uint32_t n_edges = 0, p_beg = 0, p_cnt = 0, n_pass = 0;
+        bool later = false;
+        int he = 0, s = -1;
         uint64_t q = 0;
-        if (lane < take) {
-            const uint32_t es = W.ent_slot[o];
-            slot = es & 63u;
-            if (!W.hit[slot]) {
-                g = W.geom[o];
-                if (KIND == KIND_MIXED) circle = (es & WL_CIRCLE) != 0u;
-                if (FILT) q = W.qidx[slot];
-                bool entire = false;
-                // a circle's start node is visited only if the circle meets its box (circle_cells);
-                // a pushed quadrant's box has passed the same test
-                if (KIND == KIND_EDGE || !circle || (item & WL_NODE_MASK) == 0u || circle_box(g.x, g.y, g.z, nd.bbox))
-                    s = strongest_t<FILT>(c, nd, f, q, entire);
-                if (s >= 0 && entire) {
-                    W.hit[slot] = 1u;
-                    s = -1;
-                } else if (s >= 0 && nd.first_child >= 0) {
-                    fc = nd.first_child;
-                    m = circle ? circle_quadrants(g.x, g.y, g.z, nd.bbox) : edge_quadrants_node(g, nd.bbox);
-                    s = -1;
-                } else if (s >= 0) {
-                    // leaf: count the edge tests of its relevant Partial hazards
-                    he = (int)(nd.haz_begin + (nd.haz_info & COUNT_MASK));
-                    for (int i = s; i < he; i++) {
-                        const DevEntry e = ldg_ent(c.ent + i);
-                        if (!irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g)) {
-                            if (n_pass == 0u) {
-                                p_beg = e.edge_begin;
-                                p_cnt = e.edge_count;
-                            }
-                            n_pass++;
-                            n_edges += (e.edge_count + (uint32_t)EG - 1u) / (uint32_t)EG;
+        act = act && (nd.haz_info & COUNT_MASK) != 0u;
+        if (act && !(KIND == KIND_EDGE || !circle || (item & WL_NODE_MASK) == 0u)) act = circle_box(g.x, g.y, g.z, nd.bbox);
+        if (act) {
+            if (FILT) q = W.qidx[slot];
+            bool entire = false;
+            s = strongest_t<FILT>(c, nd, f, q, entire);
+            if (s >= 0 && entire) {
+                W.hit[slot] = 1u;
+            } else if (s >= 0 && nd.first_child >= 0) {
+                later = true;
+            } else if (s >= 0) {
+                he = (int)(nd.haz_begin + (nd.haz_info & COUNT_MASK));
+                for (int i = s; i < he; i++) {
+                    const DevEntry e = ldg_ent(c.ent + i);
+                    if (!irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g)) {
+                        if (n_pass == 0u) {
+                            p_beg = e.edge_begin;
+                            p_cnt = e.edge_count;
                         }
+                        n_pass++;
+                        n_edges += (e.edge_count + (uint32_t)EG - 1u) / (uint32_t)EG;
                     }
                 }
             }
         }
-        auto test_leaf = [&]() {                      // this lane tests the leaf's edges itself
-            bool h = false;
-            for (int i = s; i < he && !h; i++) {
-                const DevEntry e = ldg_ent(c.ent + i);
-                if (irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) || !ff_pass(e, circle, g)) continue;
-                for (uint32_t j = 0; j < e.edge_count && !h; j++) h = edge_hit(circle, g, ldg4(c.edges + e.edge_begin + j));
-            }
-            if (h) W.hit[slot] = 1u;
-        };
-        if (n_edges >= EDGE_LIMIT) {                  // more edge tests than one push carries
-            test_leaf();
-            n_edges = 0;
-        }
-        // one scan for both pushes: child counts in the low 16 bits, edge counts in the high
-        // 16; neither sum over the wave carries out of its half
-        const uint32_t packed = (uint32_t)__builtin_popcount(m) | (n_edges << 16);
-        const uint32_t incl = wave_incl_scan(packed, lane);
-        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-        const uint32_t excl = incl - packed;
-        const uint32_t n_tot = tot & 0xffffu, e_tot = tot >> 16;
-        wave_sync();                              // every lane has read its item before pushes overwrite
-        {
-            uint32_t at = base + (excl & 0xffffu);     // base + n_tot <= WL_NCAP by the choice of take
-            for (uint32_t b = m; b; b &= b - 1u)
-                W.nodes[at++] = (item & ~WL_NODE_MASK) | (uint32_t)(fc + __builtin_ctz(b));
-            nn = base + n_tot;
-        }
-        const bool fits = ne + e_tot <= WL_ECAP;
-        if (n_edges) {
-            uint32_t at = ne + (excl >> 16);
-            auto push = [&](uint32_t beg, uint32_t cnt) {
-                for (uint32_t j = 0; j < cnt; j += EG, at++) {
-                    const uint32_t k = cnt - j < (uint32_t)EG ? cnt - j : (uint32_t)EG;
-                    W.edges[at] = (beg + j) | ((k - 1u) << 29);
-                    W.edge_ent[at] = (uint8_t)o;
-                }
-            };
-            if (!fits) {
-                test_leaf();                          // edge queue full
-            } else if (n_pass == 1u) {
-                push(p_beg, p_cnt);                   // one passing entry (the common leaf): its edges from the count above
-            } else {
-                for (int i = s; i < he; i++) {
-                    const DevEntry e = ldg_ent(c.ent + i);
-                    if (!irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g)) push(e.edge_begin, e.edge_count);
-                }
+        // a leaf of several passing entries is left to run() as well
+        later = later || n_edges >= EDGE_LIMIT || n_pass > 1u;
+        if (later) n_edges = 0;
+        const uint32_t incl = wave_incl_scan(n_edges, lane);
+        const uint32_t e_tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        const bool fits = ne + e_tot <= ECAP;
+        if (n_edges && fits) {
+            uint32_t at = ne + incl - n_edges;
+            for (uint32_t j = 0; j < p_cnt; j += EG, at++) {
+                const uint32_t k = p_cnt - j < (uint32_t)EG ? p_cnt - j : (uint32_t)EG;
+                W.edges[at] = (p_beg + j) | ((k - 1u) << 29);
+                W.edge_ent[at] = (uint8_t)(item >> 24);
             }
         }
         if (fits) ne += e_tot;
+        push_root(later || (n_edges != 0u && !fits), item);
     }
-    wave_sync();
-}
+
+    __device__ __forceinline__ void run() {
+        while (nn + ne != 0u) {
+            wave_sync();                              // pushes and hit flags of the last step are visible
+            if (ne >= 64u || nn == 0u) {
+                // edge step: an item's edges are read before any is evaluated
+                const uint32_t take = ne < 64u ? ne : 64u;
+                const uint32_t at = lane < take ? ne - 1u - lane : 0u;
+                const uint32_t eo = W.edge_ent[at];
+                const uint32_t v = lane < take ? W.edges[at] : 0u;
+                const uint32_t e0 = v & WL_EDGE_INDEX, cnt = (v >> 29) + 1u;
+                float4 hedge[EG];
+#pragma unroll
+                for (int k = 0; k < EG; k++) hedge[k] = ldg4(c.edges + e0 + ((uint32_t)k < cnt ? (uint32_t)k : 0u));
+                if (lane < take) {
+                    const uint32_t es = W.ent_slot[eo];
+                    const uint32_t slot = es & 63u;
+                    if (!W.hit[slot]) {
+                        const bool circle = KIND == KIND_CIRCLE || (KIND == KIND_MIXED && (es & WL_CIRCLE) != 0u);
+                        const float4 gm = W.geom[eo];
+                        bool h = false;
+#pragma unroll
+                        for (int k = 0; k < EG; k++) h = h || ((uint32_t)k < cnt && edge_hit(circle, gm, hedge[k]));
+                        if (h) W.hit[slot] = 1u;
+                    }
+                }
+                ne -= take;
+                continue;
+            }
+            // node step.  An item pushes at most 4 children, 3 more slots than it frees, so taking t
+            // items grows the queue by at most 3t: steps take no more than keeps WL_RESERVE slots
+            // free.  Within the reserve, single-item steps walk depth-first, which grows the queue by
+            // at most 3 per level below where the walk began; the reserve covers the deepest tree.
+            // The queue therefore never overflows and every step makes progress.
+            uint32_t take = 1u;
+            if (nn + 3u + WL_RESERVE <= NCAP) {
+                const uint32_t room = (NCAP - WL_RESERVE - nn) / 3u;
+                take = nn < 64u ? nn : 64u;
+                take = take < room ? take : room;
+            }
+            const uint32_t base = nn - take;
+            const uint32_t item = lane < take ? W.nodes[nn - 1u - lane] : 0u;
+            const uint32_t o = item >> 24;
+            const DevNode nd = ldg_node(c.nodes + (item & WL_NODE_MASK));
+            uint32_t m = 0, n_edges = 0, slot = 0;
+            uint32_t p_beg = 0, p_cnt = 0, n_pass = 0;    // a leaf's first passing entry's edges; passing entries
+            int fc = 0, s = -1, he = 0;
+            bool circle = KIND == KIND_CIRCLE;
+            float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            uint64_t q = 0;
+            if (lane < take) {
+                const uint32_t es = W.ent_slot[o];
+                slot = es & 63u;
+                if (!W.hit[slot]) {
+                    g = W.geom[o];
+                    if (KIND == KIND_MIXED) circle = (es & WL_CIRCLE) != 0u;
+                    if (FILT) q = W.qidx[slot];
+                    bool entire = false;
+                    // a circle's start node is visited only if the circle meets its box (circle_cells);
+                    // a pushed quadrant's box has passed the same test
+                    if (KIND == KIND_EDGE || !circle || (item & WL_NODE_MASK) == 0u || circle_box(g.x, g.y, g.z, nd.bbox))
+                        s = strongest_t<FILT>(c, nd, f, q, entire);
+                    if (s >= 0 && entire) {
+                        W.hit[slot] = 1u;
+                        s = -1;
+                    } else if (s >= 0 && nd.first_child >= 0) {
+                        fc = nd.first_child;
+                        m = circle ? circle_quadrants(g.x, g.y, g.z, nd.bbox) : edge_quadrants_node(g, nd.bbox);
+                        s = -1;
+                    } else if (s >= 0) {
+                        // leaf: count the edge tests of its relevant Partial hazards
+                        he = (int)(nd.haz_begin + (nd.haz_info & COUNT_MASK));
+                        for (int i = s; i < he; i++) {
+                            const DevEntry e = ldg_ent(c.ent + i);
+                            if (!irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g)) {
+                                if (n_pass == 0u) {
+                                    p_beg = e.edge_begin;
+                                    p_cnt = e.edge_count;
+                                }
+                                n_pass++;
+                                n_edges += (e.edge_count + (uint32_t)EG - 1u) / (uint32_t)EG;
+                            }
+                        }
+                    }
+                }
+            }
+            // more edge tests than one push carries: this lane tests the leaf's edges itself
+            bool inl = n_edges >= EDGE_LIMIT;
+            if (inl) n_edges = 0;
+            // one scan for both pushes: child counts in the low 16 bits, edge counts in the high
+            // 16; neither sum over the wave carries out of its half
+            const uint32_t packed = (uint32_t)__builtin_popcount(m) | (n_edges << 16);
+            const uint32_t incl = wave_incl_scan(packed, lane);
+            const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            const uint32_t excl = incl - packed;
+            const uint32_t n_tot = tot & 0xffffu, e_tot = tot >> 16;
+            wave_sync();                              // every lane has read its item before pushes overwrite
+            {
+                uint32_t at = base + (excl & 0xffffu);     // base + n_tot <= NCAP by the choice of take
+                for (uint32_t b = m; b; b &= b - 1u)
+                    W.nodes[at++] = (item & ~WL_NODE_MASK) | (uint32_t)(fc + __builtin_ctz(b));
+                nn = base + n_tot;
+            }
+            const bool fits = ne + e_tot <= ECAP;
+            inl = inl || (!fits && n_edges != 0u);        // or the edge queue is full
+            if (n_edges && !inl) {
+                uint32_t at = ne + (excl >> 16);
+                // one passing entry (the common leaf): its edges from the count above
+                const bool one = n_pass == 1u;
+                for (int i = one ? he - 1 : s; i < he; i++) {
+                    uint32_t beg = p_beg, cnt = p_cnt;
+                    if (!one) {
+                        const DevEntry e = ldg_ent(c.ent + i);
+                        beg = e.edge_begin;
+                        cnt = !irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) && ff_pass(e, circle, g) ? e.edge_count : 0u;
+                    }
+                    for (uint32_t j = 0; j < cnt; j += EG, at++) {
+                        const uint32_t k = cnt - j < (uint32_t)EG ? cnt - j : (uint32_t)EG;
+                        W.edges[at] = (beg + j) | ((k - 1u) << 29);
+                        W.edge_ent[at] = (uint8_t)o;
+                    }
+                }
+            }
+            if (inl) {
+                bool h = false;
+                for (int i = s; i < he && !h; i++) {
+                    const DevEntry e = ldg_ent(c.ent + i);
+                    if (irrel<FILT>(f, q, e.slot_flags & SLOT_MASK) || !ff_pass(e, circle, g)) continue;
+                    for (uint32_t j = 0; j < e.edge_count && !h; j++) h = edge_hit(circle, g, ldg4(c.edges + e.edge_begin + j));
+                }
+                if (h) W.hit[slot] = 1u;
+            }
+            if (fits) ne += e_tot;
+        }
+        wave_sync();
+    }
+};
 
 // Hazard-polygon point-in-polygon (simple_polygon.rs:255-292) over the hazard's full shape.
 __device__ __forceinline__ bool pip_hazard(const CdeView& c, uint32_t slot, float px, float py) {

@@ -270,7 +270,7 @@ JG_HD uint32_t grid_index(float off, float scale, float top) { return (uint32_t)
 // strongest relevant hazard is Entire) with circle_box(T).  That test is hereditary in f32: the
 // distance per axis to a box inside another is no smaller, and subtraction, squares, the sum and
 // the comparison are monotone, so circle_box(T) holds for every node above T too, and the descent
-// reaches T (the argument of start_node_below covers the relevant hazards on the way).  A node's
+// reaches T (the argument of edge_cells covers the relevant hazards on the way).  A node's
 // box is met through its point nearest to the centre; the nodes below that hold this point have
 // the same nearest point, hence the same distance.  So it is enough to start at the nodes of
 // all cells that can hold such a point, each visited only if circle_box holds for it.  The point
@@ -300,6 +300,64 @@ JG_HD CircleCells circle_cells(const CellGrid& g, uint32_t level, float4 root, f
     o.y1 = y1 >> s;
     return o;
 }
+// The cell that strictly holds a box: (ix, iy) of level l, the deepest of the even grid's cells that
+// the box, widened by the grid's margin, lies in.  A cell's bounds as the tree builds them,
+// midpoints of midpoints, are a few ulps off the even grid, so the box lies strictly on one side
+// of every midline above the cell.  (l = 0 without a grid.)
+struct HoldingCell {
+    uint32_t l, ix, iy;
+};
+JG_HD HoldingCell holding_cell(const CellGrid& g, uint32_t level, float4 root, float4 b) {
+    const float top = (float)((1u << level) - 1u);
+    const uint32_t x0 = grid_index(b.x - g.eps - root.x, g.sx, top), x1 = grid_index(b.z + g.eps - root.x, g.sx, top);
+    const uint32_t y0 = grid_index(b.y - g.eps - root.y, g.sy, top), y1 = grid_index(b.w + g.eps - root.y, g.sy, top);
+    const uint32_t d = (x0 ^ x1) | (y0 ^ y1);
+    const uint32_t s = !(g.sx > 0.0f) ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
+    return HoldingCell{level - s, x0 >> s, y0 >> s};
+}
+
+// The start cells of the descent of an edge with bounding box b, within the root box: the cell that
+// strictly holds it, or, deeper, the two cells of one level that share a side which the edge
+// crosses, (x0, y0) and (x1, y1) of level l (equal for one cell).
+//
+// QTNode::collides reaches the deepest nodes on the paths to these cells and no others beside or
+// above them matter.  Every hazard present below a node is an entry of it (qt_node.rs:39-81:
+// hazards reach children by constrict, and an Entire hazard is Entire in every quadrant,
+// qt_hazard.rs:58), and Entire entries come first (qt_hazard_vec.rs), so along a path: an
+// ancestor without relevant hazards leaves the node none either, and one whose strongest
+// relevant hazard is Entire leaves it Entire.  And the visits on the way push just the path's
+// next node (collides_with_quadrants, qt_traits.rs:19-106):
+//  - where the edge lies strictly inside one quadrant, the box test finds the others disjoint;
+//  - at the node whose midline is the side crossed, each endpoint lies in a quadrant of its own,
+//    which collides for that, and the other two are disjoint, as the edge lies strictly inside
+//    one half of the other axis: both paths;
+//  - below it, the edge leaves the node across that side only; its endpoint lies strictly inside the
+//    quadrant on the path, and the other three are disjoint, beyond the endpoint or the midline.
+// "Strictly" is by the margin of holding_cell, for the endpoints against the crossed side as well;
+// where it fails, one cell of a level above is taken.
+struct EdgeCells {
+    uint32_t l, x0, y0, x1, y1;
+};
+JG_HD EdgeCells edge_cells(const CellGrid& g, uint32_t level, float4 root, float4 b) {
+    const float top = (float)((1u << level) - 1u);
+    const uint32_t x0 = grid_index(b.x - g.eps - root.x, g.sx, top), x1 = grid_index(b.z + g.eps - root.x, g.sx, top);
+    const uint32_t y0 = grid_index(b.y - g.eps - root.y, g.sy, top), y1 = grid_index(b.w + g.eps - root.y, g.sy, top);
+    const uint32_t d = (x0 ^ x1) | (y0 ^ y1);
+    uint32_t s = !(g.sx > 0.0f) ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
+    EdgeCells o{level - s, x0 >> s, y0 >> s, x0 >> s, y0 >> s};
+    if (s != 0u && g.sx > 0.0f) {
+        const uint32_t x2 = grid_index(b.x + g.eps - root.x, g.sx, top), x3 = grid_index(b.z - g.eps - root.x, g.sx, top);
+        const uint32_t y2 = grid_index(b.y + g.eps - root.y, g.sy, top), y3 = grid_index(b.w - g.eps - root.y, g.sy, top);
+        uint32_t t = 0;                       // the least shift with at most two cells, side by side
+        while (t < s && ((x1 >> t) - (x0 >> t)) + ((y1 >> t) - (y0 >> t)) > 1u) t++;
+        // across a vertical side the endpoints' x decide, across a horizontal one their y
+        const bool xs = x0 >> t != x1 >> t;
+        const bool sure = xs ? x2 >> t == x0 >> t && x3 >> t == x1 >> t : y2 >> t == y0 >> t && y3 >> t == y1 >> t;
+        if (t < s && sure) o = EdgeCells{level - t, x0 >> t, y0 >> t, x1 >> t, y1 >> t};
+    }
+    return o;
+}
+
 // circle.rs:109-113 via edge.rs:63-87,153-159  Circle–Edge
 JG_HD bool circle_edge(float cx, float cy, float rad, float4 e) {
     float a = cx - e.x, b = cy - e.y, c = e.z - e.x, d = e.w - e.y;

@@ -228,18 +228,19 @@ def test_shared_interval_quadrant_forms(tmp_path):
         assert ok == "ok" and int(on_mid) > 100000
 
 
-def test_circle_start_cells(tmp_path):
-    """The nodes a circle's descent may start at (circle_cells in jg_geom.hpp) reach exactly the
-    leaves that the descent from the root reaches (tests/circle_cells_check.cpp)."""
+def test_start_cells(tmp_path):
+    """The nodes that the descents of circles and edges may start at (circle_cells and edge_cells in
+    jg_geom.hpp) reach exactly the leaves that the descents from the root reach, and the
+    virtual root's path passes the cell that holds a box (tests/start_cells_check.cpp)."""
     import os
     import subprocess
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    exe = tmp_path / "circle_cells_check"
+    exe = tmp_path / "start_cells_check"
     subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
-                    "-I/opt/rocm/include", os.path.join(root, "tests", "circle_cells_check.cpp"), "-o", str(exe)],
+                    "-I/opt/rocm/include", os.path.join(root, "tests", "start_cells_check.cpp"), "-o", str(exe)],
                    check=True, capture_output=True)
     for seed in (1, 2):
         out = subprocess.run([str(exe), str(seed), "4000"], capture_output=True, text=True)
         assert out.returncode == 0, out.stdout + out.stderr
-        ok, leaves, on = out.stdout.split()
-        assert ok == "ok" and int(leaves) > 10000 and int(on) > 30000
+        ok, leaves, on, two = out.stdout.split()
+        assert ok == "ok" and int(leaves) > 10000 and int(on) > 30000 and int(two) > 5000
