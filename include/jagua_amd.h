@@ -252,10 +252,10 @@ typedef struct {
 } jg_query_set;
 
 typedef struct {
-    uint32_t chunk;                       /* queries per work unit: 16, 32, 64 (0 = 64) */
-    uint32_t workgroups;                  /* persistent one-wavefront workgroups (0 = 16 per compute unit) */
-    uint32_t lanes_per_query;             /* 0 = per item: its vertex count rounded up to a power
-                                             of two, 8..32 */
+    uint32_t chunk;                       /* queries per work unit: 16, 32, 64 (0 = 64, 32 in a small launch) */
+    uint32_t workgroups;                  /* one-wavefront workgroups (0 = one per work unit in the surrogate
+                                             stage, 20 per compute unit in the polygon stage) */
+    uint32_t lanes_per_query;             /* 0 = per item, 8..64 by its vertex count, 64 in a small launch */
     uint32_t flags;                       /* JG_QUERY_* */
     uint32_t stages;                      /* 0 or 2: surrogate and polygon stages as two kernels,
                                              survivors passed in groups of one polygon pass;

@@ -13,7 +13,7 @@
 // The default schedule is these two kernels.  k_fused runs both stages of a work unit in one
 // wave instead: no survivor queue, but a unit with many survivors keeps its wave busy long
 // after the others finish; the autotuner weighs it.  Units are ordered by item size (largest
-// first).  Work is claimed from 8 interleaved streams of counters, never from one address.
+// first).  Work is claimed from interleaved streams of counters, never from one address.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -166,9 +166,11 @@ __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict
     __shared__ SurrLds lds;
     // the polygon stage of this launch claims groups after this kernel: clear its claim counters
     if (blockIdx.x == 0 && lane < N_STREAMS) counters[C_STREAM0 + STREAM_STRIDE * lane] = 0u;
-    uint32_t ux = blockIdx.x & (N_STREAMS - 1u), utried = 0;
+    if (blockIdx.x == 0 && lane == 0) atomicAdd(&counters[C_EPOCH], 1u);
+    const uint32_t p = ldg1(counters + C_EPOCH + 1u) & 1u;
+    Claims claims;
     for (;;) {
-        const uint32_t u = claim_next(counters, C_USTREAM0, ux, utried, n_units, lane);
+        const uint32_t u = wave_bcast(claims.next(counters, C_USTREAM0, n_units, lane));
         if (u >= n_units) return;
         const Unit un = units[u];
         const uint64_t todo = surrogate_unit<FILT, KIND>(sets[un.set], un, lds, m6, status, lane);
@@ -176,9 +178,9 @@ __global__ __launch_bounds__(WAVE, 5) void k_surrogate(const SetDesc* __restrict
             // one survivor group per polygon-stage pass (64 / G queries)
             const uint32_t per = 64u / sets[un.set].lanes;
             const uint32_t n_g = ((uint32_t)__builtin_popcountll(todo) + per - 1u) / per;
-            // the unit's stream (u mod 8) appends to its own region of the group array
+            // the unit's stream appends to its own region of the group array
             const uint32_t xs = u & (N_STREAMS - 1u);
-            const uint32_t g0 = gbase[xs] + atomicAdd(&counters[C_GCOUNT0 + STREAM_STRIDE * xs], n_g);
+            const uint32_t g0 = gbase[xs] + atomicAdd(&counters[C_GCOUNT0 + STREAM_STRIDE * (N_STREAMS * p + xs)], n_g);
             uint64_t rest = todo;
             for (uint32_t j = 0; j < n_g; j++) {
                 uint64_t r = rest;
@@ -411,25 +413,32 @@ __device__ __forceinline__ void poly_loop(const SetDesc* __restrict__ sets, uint
                                           const Group* __restrict__ groups, const uint32_t* __restrict__ gbase,
                                           const float* __restrict__ m6, uint8_t* __restrict__ status, WaveLds& lds) {
     const uint32_t lane = threadIdx.x;
-    // the surrogate stage of this launch is done: clear its unit-claim counters for the next
-    if (blockIdx.x == 0 && lane < N_STREAMS) counters[C_USTREAM0 + STREAM_STRIDE * lane] = 0u;
-    // stream x holds the groups its units appended; a wave drains its own stream, then the next
-    uint32_t x = blockIdx.x & (N_STREAMS - 1u);
-    for (uint32_t tried = 0; tried < N_STREAMS;) {
-        const uint32_t n_x = __atomic_load_n(&counters[C_GCOUNT0 + STREAM_STRIDE * x], __ATOMIC_RELAXED);
-        uint32_t j = 0;
-        if (lane == 0) j = atomicAdd(&counters[C_STREAM0 + STREAM_STRIDE * x], 1u);
-        j = wave_bcast(j);
-        if (j >= n_x) {
-            x = (x + 1u) & (N_STREAMS - 1u);
-            tried++;
-            continue;
-        }
-        const Group gr = groups[gbase[x] + j];
+    // the surrogate stage of this launch is done: clear its unit-claim counters for the next, and the
+    // group counts of the other parity.  Lane y finds where region y of the list of groups ends
+    // (kept in LDS, so that no register holds it over the pass)
+    __shared__ uint32_t ends[N_STREAMS];
+    const uint32_t p = (ldg1(counters + C_EPOCH) - 1u) & 1u;
+    uint32_t end = lane < N_STREAMS ? ldg1(counters + C_GCOUNT0 + STREAM_STRIDE * (N_STREAMS * p + lane)) : 0u;
+    if (blockIdx.x == 0 && lane < N_STREAMS) {
+        counters[C_USTREAM0 + STREAM_STRIDE * lane] = 0u;
+        counters[C_GCOUNT0 + STREAM_STRIDE * (N_STREAMS * (p ^ 1u) + lane)] = 0u;
+    }
+    if (blockIdx.x == 0 && lane == 0) atomicAdd(&counters[C_EPOCH + 1u], 1u);
+    end = wave_incl_scan(end, lane);
+    if (lane < N_STREAMS) ends[lane] = end;
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)end, N_STREAMS - 1);
+    wave_sync();
+    Claims claims;
+    for (;;) {
+        const uint32_t v = wave_bcast(claims.next(counters, C_STREAM0, n, lane));
+        if (v >= n) return;
+        // group v of the list: region y, at v less the end of the region before
+        const uint32_t e = ends[lane & (N_STREAMS - 1u)];
+        const uint32_t y = (uint32_t)__builtin_popcountll(__ballot(lane < N_STREAMS && e <= v));
+        const uint32_t before = y ? (uint32_t)__builtin_amdgcn_readlane((int)e, (int)y - 1) : 0u;
+        const Group gr = groups[wave_bcast(gbase[y] + (v - before))];
         poly_queries<FILT>(sets[gr.set], gr.q0, gr.mask, lds, m6, status, lane);
     }
-    // every wave has read the group counts once the last one is out
-    if (last_wave_out(counters, lane) && lane < N_STREAMS) counters[C_GCOUNT0 + STREAM_STRIDE * lane] = 0u;
 }
 
 // k_poly is bound by VALU issue (80% of SIMD cycles, half the lanes active), most of it the set-up and
@@ -468,9 +477,9 @@ __device__ __forceinline__ void fused_loop(const SetDesc* __restrict__ sets, con
                                            const float* __restrict__ m6, uint8_t* __restrict__ status,
                                            WaveLds& lds) {
     const uint32_t lane = threadIdx.x;
-    uint32_t ux = blockIdx.x & (N_STREAMS - 1u), utried = 0;
+    Claims claims;
     for (;;) {
-        const uint32_t u = claim_next(counters, C_USTREAM0, ux, utried, n_units, lane);
+        const uint32_t u = wave_bcast(claims.next(counters, C_USTREAM0, n_units, lane));
         if (u >= n_units) break;
         const Unit un = units[u];
         const SetDesc& sd = sets[un.set];
@@ -623,6 +632,8 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
         if (s.cde->img.cap_edges > WL_MAX_EDGES)
             return fail(JG_ERR_CAPACITY, "engine image of more than 2^29 hazard edges in a batched plan");
     }
+    uint64_t n_all = 0;
+    for (auto& s : sets) n_all += s.count;
     std::vector<SetDesc> sd(sets.size());
     bool any_filter = false, any_pole = false, any_pier = false;
     L.max_slot_words = 1;
@@ -643,10 +654,14 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
         sd[i].first = s.first;
         uint32_t lanes = cfg.lanes_per_query;
         if (lanes == 0) {
-            // the vertex count rounded up to a power of two, 8..32: items above 32 vertices run
-            // two queries per pass, which measured faster than one query on 64 lanes
-            lanes = 8;
-            while (lanes < s.item->poly.n() && lanes < 32u) lanes <<= 1;
+            // by vertices in a large launch: us per step at up to 32 lanes (the vertices rounded up) / at
+            // these / at 64 for all above 32, 552 / 539 / 592 (2000-item sheet), 363 / 333 / 345
+            // (concave items of 300 vertices at the mean).  A launch with waves to spare, a query
+            // or less for each after the surrogate stage: the whole wave, as its time is a pass's
+            // (32000 queries of 64 items of 8-512 vertices: 93 -> 81 us).
+            const uint32_t v = s.item->poly.n();
+            lanes = v <= 16u ? 8u : v <= 64u ? 16u : v <= 384u ? 32u : 64u;
+            if (n_all <= (uint64_t)n_cus * 160u) lanes = 64u;
         }
         uint32_t pow2 = 1;
         while (pow2 < lanes && pow2 < 64u) pow2 <<= 1;
@@ -662,7 +677,8 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
     // work units: sets in decreasing item size, `chunk` queries each (16, 32 or 64; 64 packs
     // 128 pole entities into one surrogate traversal; smaller units shorten the fused kernel's
     // tail)
-    const uint32_t uq = cfg.chunk == 0 ? 64u : cfg.chunk <= 16u ? 16u : cfg.chunk <= 32u ? 32u : 64u;
+    // (32 by default in a launch with waves to spare: 16000 queries of 64-vertex items 63 -> 55 us)
+    const uint32_t uq = cfg.chunk == 0 ? (n_all <= (uint64_t)n_cus * 160u ? 32u : 64u) : cfg.chunk <= 16u ? 16u : cfg.chunk <= 32u ? 32u : 64u;
     std::vector<size_t> order(sets.size());
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
@@ -678,7 +694,7 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
     L.o_units = (sizeof(SetDesc) * sd.size() + 255) & ~(size_t)255;
     L.o_ctr = (L.o_units + sizeof(Unit) * units.size() + 255) & ~(size_t)255;
     L.o_gbase = L.o_ctr + 4u * N_COUNTER_WORDS;
-    // one group per polygon-stage pass at most; unit u's groups go to the region of stream u mod 8
+    // one group per polygon-stage pass at most; unit u's groups go to the region of its stream
     uint64_t stream_groups[N_STREAMS] = {};
     for (size_t u = 0; u < units.size(); u++) {
         const uint32_t per = 64u / sd[units[u].set].lanes;
@@ -699,7 +715,9 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
     std::memcpy(host.data() + L.o_gbase, gbase, sizeof(gbase));
     // one wavefront per workgroup, each taking one work unit (or survivor group) at a time
     const uint32_t want = cfg.workgroups ? cfg.workgroups : n_cus * 20u;
-    L.grid_s = std::max<uint32_t>(1u, std::min<uint32_t>(want, L.n_units));
+    // a surrogate unit is short: one workgroup each, dispatched by the hardware, costs less than claims
+    // (465 -> 455 us per benchmark step), up to a million
+    L.grid_s = std::max<uint32_t>(1u, std::min<uint32_t>(cfg.workgroups || L.stages == 1u ? want : 1u << 20, L.n_units));
     L.grid_p = std::max<uint32_t>(1u, (uint32_t)std::min<uint64_t>(want, max_groups));
     return JG_OK;
 }

@@ -705,9 +705,9 @@ __global__ __launch_bounds__(WAVE, CL_WAVES) void k_collect_units(const SetDesc*
                                                        uint32_t* __restrict__ keys, uint64_t* __restrict__ ovf) {
     __shared__ CollectLds lds;
     const uint32_t lane = threadIdx.x;
-    uint32_t ux = blockIdx.x & (N_STREAMS - 1u), utried = 0;
+    Claims claims;
     for (;;) {
-        const uint32_t u = claim_next(counters, C_USTREAM0, ux, utried, n_units, lane);
+        const uint32_t u = wave_bcast(claims.next(counters, C_USTREAM0, n_units, lane));
         if (u >= n_units) return;
         const Unit un = units[u];
         const uint32_t si = wave_bcast(un.set);
@@ -728,7 +728,7 @@ jg_status collect_launch(const TableLayout& L, uint8_t* base, const float* d_m6,
     const SetDesc* sets = (const SetDesc*)base;
     const Unit* units = (const Unit*)(base + L.o_units);
     hipLaunchKernelGGL(k_collect_reset, dim3(1), dim3(64), 0, stream, counters);
-    const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(n_cus * 4u * CL_WAVES, L.n_units));
+    const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(1u << 20, L.n_units));   // a workgroup per unit, up to a million
     hipLaunchKernelGGL(k_collect_units, dim3(grid), dim3(WAVE), 0, stream, sets, units, L.n_units, counters, d_m6,
                        d_keys ? cap : 0u, d_count, d_hash, d_keys, ovf);
     jg_status st = hip_check(hipGetLastError(), "batched collection launch");

@@ -34,24 +34,36 @@ struct Group {             // 16 B: surviving queries q0 + i for the set bits i 
     uint64_t mask;
 };
 
-// Work is claimed from 8 streams, each with its own counters on their own 128-byte lines:
+// Work is shared out over 16 streams, each with its own counters on their own 128-byte lines:
 // thousands of waves taking work with atomics on a single address queue behind each other
 // (measured: 1.81 ms against 1.30 ms per configuration-2 step for the survivor groups alone).
-//   unit stream x:  units x + 8 j; counter C_USTREAM0 + 32 x counts the units taken
-//   group stream x: the survivor groups of the units of unit stream x, in their own region of
-//                   the group array (base gbase[x]); C_GCOUNT0 + 32 x counts the groups
-//                   appended, C_STREAM0 + 32 x the groups taken
-// A wave starts on stream blockIdx.x mod 8 and moves to the next one as each runs dry.
+// Items x + 16 j of a list, work units or survivor groups, are stream x's; a wave claims from its own
+// stream (workgroup index mod 16) alone, and a launch of at least as many workgroups as items takes
+// them without a claim.  Looking at the other streams once the own one is dry costs more than the
+// balance it brings, as thousands of waves then end with atomics or loads on the same few lines:
+// us per step without / with a try of each stream / with a look at all counters first, 488 / 543 /
+// 647 on the benchmark's 2000-item sheet, 275 / 337 / 401 on concave items.  For that reason no
+// wave counts itself out either (a batch of 6400 queries took 111 us with both, 70 without).  8 / 16 /
+// 32 streams: 471 / 465 / 472.
+//   C_USTREAM0 + 32 x counts the units claimed from stream x, C_STREAM0 + 32 x the groups.
+//   The survivor groups of the units of unit stream y are appended to their own region of the group
+//   array (base gbase[y]); C_GCOUNT0 + 32 (16 p + y) counts them in the launches of parity p.
+//   The regions one after another are the list of groups.
+//   C_EPOCH counts the surrogate stages, C_EPOCH + 1 the polygon stages of the table.  Each stage
+//   takes the parity from the other's count, which stands still meanwhile; the polygon stage
+//   clears the other parity's counts, for the next launch.
 // C_OVERFLOW counts the queries the batched collection hands to the per-query collector;
 // C_DONE counts the waves of a launch that have finished (the last one clears counters).
-// Every launch sequence leaves all counters at zero for the next, and a new table starts so.
-constexpr uint32_t N_STREAMS = 8, STREAM_STRIDE = 32;
+// Every launch sequence leaves the table's counters ready for the next, and a new table, all zero,
+// is.
+constexpr uint32_t N_STREAMS = 16, STREAM_STRIDE = 32;
 constexpr uint32_t C_STREAM0 = 0;
 constexpr uint32_t C_USTREAM0 = C_STREAM0 + STREAM_STRIDE * N_STREAMS;
 constexpr uint32_t C_GCOUNT0 = C_USTREAM0 + STREAM_STRIDE * N_STREAMS;
-constexpr uint32_t C_OVERFLOW = C_GCOUNT0 + STREAM_STRIDE * N_STREAMS;
+constexpr uint32_t C_OVERFLOW = C_GCOUNT0 + 2u * STREAM_STRIDE * N_STREAMS;
 constexpr uint32_t C_DONE = C_OVERFLOW + STREAM_STRIDE;
-constexpr uint32_t N_COUNTER_WORDS = C_DONE + STREAM_STRIDE;
+constexpr uint32_t C_EPOCH = C_DONE + STREAM_STRIDE;
+constexpr uint32_t N_COUNTER_WORDS = C_EPOCH + STREAM_STRIDE;
 
 // The calling wave's exit from a launch of gridDim.x one-wave workgroups: true in the last
 // wave to leave, once every other wave has left (C_DONE is then back at zero).
@@ -67,7 +79,7 @@ __device__ __forceinline__ bool last_wave_out(uint32_t* counters, uint32_t lane)
 constexpr uint32_t WAVE = 64;
 
 // The device table of a batched launch, in one buffer: set descriptors, work units, the claim
-// counters, the survivor-group region bases of the 8 streams and the survivor groups.
+// counters, the survivor-group region bases of the streams and the survivor groups.
 struct TableLayout {
     size_t o_units = 0, o_ctr = 0, o_gbase = 0, o_grp = 0, total = 0;
     uint32_t n_units = 0, grid_s = 0, grid_p = 0;
@@ -92,21 +104,29 @@ __device__ __forceinline__ T wave_bcast(T v) {
     return (T)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-// The next item of n from 8 interleaved streams (item x + 8 j in stream x, counters from word
-// base on): the wave's stream x first, then the following ones as they drain; n when all are.
-__device__ __forceinline__ uint32_t claim_next(uint32_t* counters, uint32_t base, uint32_t& x, uint32_t& tried,
-                                               uint32_t n, uint32_t lane) {
-    while (tried < N_STREAMS) {
-        uint32_t j = 0;
-        if (lane == 0) j = atomicAdd(&counters[base + STREAM_STRIDE * x], 1u);
-        j = __builtin_amdgcn_readfirstlane(j);
-        const uint64_t i = (uint64_t)x + (uint64_t)N_STREAMS * j;
-        if (i < n) return (uint32_t)i;
-        x = (x + 1u) & (N_STREAMS - 1u);
-        tried++;
+// A wave's items of a list of n, counters from word base on: the next item's index, n when there is
+// none for this wave.  Every item is taken: its stream's workgroups claim until the stream is dry,
+// and a launch of fewer workgroups than streams goes through all streams.
+struct Claims {
+    uint32_t x, tried;
+    bool fresh;                                   // nothing has been taken yet
+    __device__ __forceinline__ Claims() : x(blockIdx.x & (N_STREAMS - 1u)), tried(0u), fresh(true) {}
+    __device__ __forceinline__ uint32_t next(uint32_t* counters, uint32_t base, uint32_t n, uint32_t lane) {
+        if (n <= gridDim.x) {                     // a workgroup per item
+            const bool mine = fresh && blockIdx.x < n;
+            fresh = false;
+            return mine ? blockIdx.x : n;
+        }
+        for (;;) {
+            uint32_t t = 0;
+            if (lane == 0) t = atomicAdd(&counters[base + STREAM_STRIDE * x], 1u);
+            const uint64_t i = (uint64_t)x + (uint64_t)N_STREAMS * (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+            if (i < n) return (uint32_t)i;
+            if (gridDim.x >= N_STREAMS || ++tried == N_STREAMS) return n;
+            x = (x + 1u) & (N_STREAMS - 1u);
+        }
     }
-    return n;
-}
+};
 
 // Sum of v over the G lanes of this lane's aligned group (G a power of two <= 64).
 __device__ __forceinline__ int group_sum_i32(int v, uint32_t G) {

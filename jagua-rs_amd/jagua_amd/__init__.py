@@ -514,9 +514,10 @@ class Graph:
 class QueryPlan:
     """Batched persistent form: many (engine, item, transform range) sets in one launch.
 
-    Schedule (jg_plan_config): chunk = queries per work unit (16, 32, 64; 0 = 64); workgroups
-    = persistent one-wave workgroups (0 = 16 per compute unit); lanes_per_query = lanes per
-    query in the polygon stage (0 = per item, 8..32); stages = 0 or 2 for two kernels (the
+    Schedule (jg_plan_config): chunk = queries per work unit (16, 32, 64; 0 = 64, 32 in a small
+    launch); workgroups = one-wave workgroups (0 = one per unit in the surrogate stage, 20 per
+    compute unit in the polygon stage); lanes_per_query = lanes per query in the polygon stage
+    (0 = per item, 8..64 by its vertex count, 64 in a small launch); stages = 0 or 2 for two kernels (the
     surrogate stage, then the polygon stage over one-pass survivor groups), 1 for one kernel
     running both stages of a unit."""
 
