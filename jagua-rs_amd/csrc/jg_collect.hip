@@ -1,12 +1,12 @@
 // Batched hazard collection (jg_plan_collect): the hazard set of every query of a plan, as
 // ci_bench composes it (lbf/benches/ci_bench.rs:56-69): collect_surrogate_collisions
-// (cd_engine.rs:296-310) then collect_poly_collisions (cd_engine.rs:261-289), in persistent
-// one-wave workgroups that claim the plan's work units.
+// (cd_engine.rs:296-310) then collect_poly_collisions (cd_engine.rs:261-289), in one-wave
+// workgroups that take the plan's work units; and jg_collect_batch, one set without a plan.
 //
-// A wave collects CP queries of a unit at a time.  All their entities (ff poles and piers from
-// the root, query edges from the first collecting node of their root path below the query's
-// virtual root, collect_start_cells) share one wave traversal in the manner of the detection's
-// (node visits and edge tests queued in LDS, 64 per step), with
+// A wave collects CP queries of a unit at a time.  All their entities (ff poles and query edges,
+// each from the first collecting nodes on the paths to its cells, collect_start, and piers from the
+// root) share one wave traversal in the manner of the detection's (node visits and edge tests
+// queued in LDS, 64 per step), with
 // QTNode::collect_collisions (qt_node.rs:151-191) as the visit: a node whose active edges number
 // at most cd_threshold, or a leaf, inserts its Entire hazards and queues edge tests for its
 // Partial hazards; other nodes queue their colliding quadrants.  Each query's collector is a
@@ -25,11 +25,15 @@
 //    widened box meets the query's bbox.  Those candidates (up to NC) are listed per query when
 //    the pass starts, with each edge's mask of candidates its box meets; a visit is skipped
 //    once every candidate of its edge's mask is in the set.  The skip reads only LDS.
-//  - ff poles and piers descend from the root: a visit to a node of at most PRUNE_MAX entries
-//    is skipped when no entry outside the set may be collected by the entity's box.
+//  - ff poles and piers: a visit to a node of at most PRUNE_MAX entries is skipped when
+//    no entry outside the set may be collected by the entity's box.
 // The candidates also hold every hazard the containment loop can add (it needs a bbox
 // relation, or the exterior), so that loop runs over them.  On the configuration-2 layout
-// the skip takes the oracle's 525 node visits per query to about 196, and the start nodes to 78.
+// the skip takes the oracle's 525 node visits per query to about 196, and the start nodes to 78
+// and fewer.  Bound by VALU issue; 262144 queries of 32 items over the 2000-item sheet: 2195 ->
+// 2029 us with the start nodes found by one grid computation, two for an edge across a cell side
+// and up to four for a pole (from the root before), 1940 at 5 waves per SIMD, where fewer
+// registers spill, than at 6, and 1857 with the LDS that leaves given to the edge-test queue.
 //
 // A query whose set outgrows the LDS list (SET_CAP slots) is handed to the per-query collector
 // (k_collect_overflow), which keeps a bit per slot.  A query with more than NC candidates skips
@@ -46,15 +50,15 @@ using namespace jg;
 
 namespace {
 
-constexpr uint32_t CL_WAVES = 6;         // waves per SIMD: VGPRs (80) and LDS per wave are sized for it
+constexpr uint32_t CL_WAVES = 5;         // waves per SIMD: VGPRs (96) and LDS per wave are sized for it
 constexpr uint32_t CL_ENT = 64;          // entities per traversal (below 256: 8-bit indices)
 constexpr uint32_t CL_NCAP = 320;        // node-visit queue entries
-static_assert(CL_NCAP >= CL_ENT + WL_RESERVE + 3u, "node queue must hold the roots and the reserve");
+static_assert(CL_NCAP >= 4u * CL_ENT + WL_RESERVE + 3u, "node queue must hold up to four start nodes per entity and the reserve");
 constexpr uint32_t CP = 8;              // queries per collection pass
 constexpr uint32_t CG = WAVE / CP;       // lanes per query in the set-up, containment and result phases
 constexpr uint32_t SET_CAP = 16;         // slots per query collector in LDS
 constexpr uint32_t NC = 8;              // candidates per query (bits of an edge's mask)
-constexpr uint32_t CE_CAP = 128;         // edge-test queue entries
+constexpr uint32_t CE_CAP = 320;         // edge-test queue entries (us at 128, 192, 256, 320: 1947, 1894, 1889, 1857)
 constexpr uint32_t CEG = 4;              // hazard edges per edge-test entry (first edge | (count - 1) << 29)
 constexpr uint32_t CE_LIMIT = 128;       // edge tests one visit pushes: fewer (also below the scan's 16 bits)
 static_assert(64u * (CE_LIMIT - 1u) < 65536u, "a wave's edge pushes must fit 16 bits");
@@ -64,7 +68,7 @@ constexpr uint32_t SURR_MASK = 0u;       // emask of a pole or pier: the node-en
 constexpr uint32_t C_EXT = 0x80000000u;  // candidate record flags: exterior hazard, Entire in the virtual root
 constexpr uint32_t C_ENTIRE = 0x40000000u;
 constexpr uint32_t C_SLOT = 0x3fffffffu;
-constexpr uint32_t VR_COLLECTS = 0x80000000u;   // vcell flag: the virtual root collects
+constexpr uint32_t VR_COLLECTS = 0x80000000u;   // vroot flag: the virtual root collects
 
 struct CollectLds {
     uint32_t nodes[CL_NCAP];             // entity << 24 | node
@@ -78,11 +82,9 @@ struct CollectLds {
     uint32_t ncand[CP];                  // candidates found (more than NC: none are used)
     uint32_t cdone[CP];                  // bit i: candidate i is in the set
     uint32_t ovf[CP];                    // per query: its set outgrew SET_CAP
-    int32_t vroot[CP];
+    uint32_t vroot[CP];                  // the virtual root | VR_COLLECTS when it collects (a leaf, or at
+                                         // most cd_threshold active edges)
     uint32_t vdepth[CP];                 // its depth
-    uint32_t vcell[CP];                  // its cell at its level, iy << 16 | ix (levels up to the tables'),
-                                         // | VR_COLLECTS when it collects (a leaf, or at most cd_threshold active edges)
-    float4 vbox[CP];                     // its box
     float mat[CP][6];                    // per query: its transformation
     float4 qbox[CP];                     // per query: its transformed bbox
     uint32_t vbeg[CP], vcnt[CP];         // its virtual root's entry range
@@ -151,53 +153,14 @@ __device__ __forceinline__ bool may_collect(const CdeView& c, uint32_t slot, flo
     return boxes_meet(eb, widened(ldg4(c.haz_bbox + slot)));
 }
 
-// The node from which a query edge with box eb, starting at node n, reaches the same visits
-// of QTNode::collect_collisions (qt_node.rs:151-191): while n is an internal node of the
-// collection (it has children and more than cd_threshold active edges) and eb lies strictly
-// inside one of its quadrants, that quadrant's child.  An edge strictly inside a quadrant
-// collides with no other quadrant (the box test of collides_with_quadrants,
-// qt_traits.rs:19-106), so the visit of n would push just that child.
-__device__ __forceinline__ uint32_t collect_start(const CdeView& c, uint32_t n, float4 eb) {
-    for (;;) {
-        const DevNode nd = ldg_node(c.nodes + n);
-        if (nd.first_child < 0 || nd.n_active_edges <= c.cd_threshold) return n;
-        const float4 r = nd.bbox;
-        const float mxm = (r.x + r.z) / 2.0f, mym = (r.y + r.w) / 2.0f;
-        const bool xh = eb.x > mxm, xl = eb.z < mxm, yh = eb.y > mym, yl = eb.w < mym;
-        if (!(xh || xl) || !(yh || yl)) return n;
-        // children in quadrant order: top right, top left, bottom left, bottom right
-        n = (uint32_t)nd.first_child + (xh ? (yh ? 0u : 3u) : (yh ? 1u : 2u));
-    }
-}
-
-// collect_start for a query edge with box eb, of a query whose virtual root vr (depth vd, box
-// vbox, cell (vx, vy) of its level) does not collect, through the cell tables: below vr the
-// edge's root path is followed arithmetically while eb lies strictly inside one quadrant (no
-// memory read), down to the tables' deepest level; that cell's entry gives the deepest node on
-// the path and the depth of the first collecting node on it (below vr, as vr does not
-// collect), and at most one more entry gives that node.  Without one, the start is the
-// deepest node, from which collect_start goes on below the tables' levels.  The path's boxes
-// below vr hold the edge: vr's box does, and eb is strictly on one side of each midline.
-__device__ __forceinline__ uint32_t collect_start_cells(const CdeView& c, float4 eb, uint32_t vr, uint32_t vd,
-                                                        float4 vbox, uint32_t vx, uint32_t vy) {
-    if (vd >= c.cell_level) return collect_start(c, vr, eb);
-    float4 r = vbox;
-    uint32_t ix = vx, iy = vy, l = vd;
-    for (; l < c.cell_level; l++) {
-        const float mxm = (r.x + r.z) / 2.0f, mym = (r.y + r.w) / 2.0f;
-        const bool xh = eb.x > mxm, xl = eb.z < mxm, yh = eb.y > mym, yl = eb.w < mym;
-        if (!(xh || xl) || !(yh || yl)) break;
-        r = make_float4(xh ? mxm : r.x, yh ? mym : r.y, xh ? r.z : mxm, yh ? r.w : mym);
-        ix = 2u * ix + (xh ? 1u : 0u);
-        iy = 2u * iy + (yh ? 1u : 0u);
-    }
-    if (l == vd) return vr;                       // eb meets a midline of vr: vr's visit starts it
-    const uint32_t e = ldg1(c.cells + ((1u << (2u * l)) - 1u) / 3u + ((iy << l) | ix));
-    const uint32_t cd = cell_cdepth(e), n = e & CELL_NODE;
-    if (cd == 15u) return l == c.cell_level ? collect_start(c, n, eb) : n;
-    if (cd == cell_depth(e)) return n;
-    const uint32_t s = l - cd;                    // the first collecting node, above the cell's node
-    return ldg1(c.cells + ((1u << (2u * cd)) - 1u) / 3u + (((iy >> s) << cd) | (ix >> s))) & CELL_NODE;
+// The node from which the descent towards cell (ix, iy) of level l may start, of an entity that visits
+// the nodes on the path to it one after another (edge_cells and circle_cells in jg_geom.hpp): the
+// first node on the path that collects, where the descent ends (QTNode::collect_collisions,
+// qt_node.rs:151-191), or the deepest node on it when none does.
+__device__ __forceinline__ uint32_t collect_start(const CdeView& c, uint32_t l, uint32_t ix, uint32_t iy) {
+    const uint32_t e = cell_entry(c, l, ix, iy), cd = cell_cdepth(e);
+    if (cd >= cell_depth(e)) return e & CELL_NODE;          // (15: none collects)
+    return cell_entry(c, cd, ix >> (l - cd), iy >> (l - cd)) & CELL_NODE;
 }
 
 __device__ __forceinline__ float4 entity_box(bool circle, float4 g) {
@@ -308,6 +271,8 @@ __device__ __forceinline__ void wave_collect(const CdeView& c, CollectLds& L, ui
             circle = (es & WL_CIRCLE) != 0u;
             g = L.geom[o];
             live = cnt > 0u;
+            // a circle's start node is visited only if the circle meets its box (circle_cells)
+            if (live && circle && (item & WL_NODE_MASK) != 0u) live = circle_box(g.x, g.y, g.z, nd.bbox);
             if (live && em == SURR_MASK && cnt <= PRUNE_MAX) live = surrogate_live(c, L, nd, cnt, qs, entity_box(circle, g));
             if (live) {
                 if (nd.first_child >= 0 && nd.n_active_edges > c.cd_threshold) {
@@ -419,7 +384,9 @@ __device__ __forceinline__ void containment_group(const CdeView& c, CollectLds& 
     }
 }
 
-// The hazard sets of queries q0 .. q0 + P - 1 of set sd (P <= CP).
+// The hazard sets of queries q0 .. q0 + P - 1 of set sd (P <= CP).  A query whose set outgrows the
+// collector is listed in ovf, or without a list (DIRECT) its count is COUNT_OVERFLOW.
+template <bool DIRECT>
 __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_index, uint32_t q0, uint32_t P,
                                              CollectLds& L, const float* __restrict__ m6, uint32_t cap,
                                              uint32_t* __restrict__ count, uint64_t* __restrict__ hash,
@@ -453,25 +420,18 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
         L.cdone[qs] = 0u;
     }
     int vr = 0;
-    uint32_t vcnt = 0, ve0 = 0, vdepth = 0, vcell = 0, vcoll = 1;
-    float4 vbox = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    uint32_t vcnt = 0, ve0 = 0, vdepth = 0, vcoll = VR_COLLECTS;
     const float4 root_bb = ldg4((const float4*)c.nodes);
     if (active) {
         vr = virtual_root_cells(c, root_bb, bb, vdepth);
         const DevNode vn = ldg_node(c.nodes + vr);
         ve0 = vn.haz_begin;
         vcnt = vn.haz_info & COUNT_MASK;
-        vbox = vn.bbox;
-        vcoll = (vn.first_child < 0 || vn.n_active_edges <= c.cd_threshold) ? 1u : 0u;
-        uint32_t ix = 0, iy = 0;
-        if (vdepth < c.cell_level) node_cell(root_bb, vbox, vdepth, ix, iy);   // (else unused)
-        vcell = (iy << 16) | ix;
+        vcoll = (vn.first_child < 0 || vn.n_active_edges <= c.cd_threshold) ? VR_COLLECTS : 0u;
     }
     if (sub == 0) {
-        L.vroot[qs] = vr;
+        L.vroot[qs] = (uint32_t)vr | vcoll;
         L.vdepth[qs] = vdepth;
-        L.vcell[qs] = vcell | (vcoll ? VR_COLLECTS : 0u);
-        L.vbox[qs] = vbox;
         L.mat[qs][0] = m.a; L.mat[qs][1] = m.b; L.mat[qs][2] = m.c;
         L.mat[qs][3] = m.d; L.mat[qs][4] = m.e; L.mat[qs][5] = m.f;
         L.qbox[qs] = bb;
@@ -540,11 +500,13 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
     uint32_t cursor = 0;
     while (cursor < total) {
         wave_sync();
-        uint32_t n = 0;
+        uint32_t n = 0, nn = 0;                   // entities and their start nodes
         while (cursor < total && n < CL_ENT) {
             const uint32_t e = cursor + lane;
             bool want = false;
-            uint32_t root = 0, em = SURR_MASK, qi = 0;
+            uint32_t em = SURR_MASK, qi = 0;
+            uint32_t start[4] = {0u, 0u, 0u, 0u};
+            bool more[4] = {true, false, false, false};
             bool circle = false;
             float4 gm = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (e < total) {
@@ -561,6 +523,14 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                         if (circle) {
                             const float2 cc = xform(mq, p.x, p.y);
                             gm = make_float4(cc.x, cc.y, p.z, 0.0f);
+                            const CircleCells cl = circle_cells(c.grid, c.cell_level, root_bb, cc.x, cc.y, p.z);
+                            start[0] = collect_start(c, cl.l, cl.x0, cl.y0);
+                            start[1] = collect_start(c, cl.l, cl.x1, cl.y0);
+                            start[2] = collect_start(c, cl.l, cl.x0, cl.y1);
+                            start[3] = collect_start(c, cl.l, cl.x1, cl.y1);
+                            more[1] = start[1] != start[0];
+                            more[2] = start[2] != start[0] && start[2] != start[1];
+                            more[3] = start[3] != start[0] && start[3] != start[1] && start[3] != start[2];
                         } else {
                             const float2 a = xform(mq, p.x, p.y), b = xform(mq, p.z, p.w);
                             gm = make_float4(a.x, a.y, b.x, b.y);
@@ -571,7 +541,8 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                         const float2 va = ldg2(it.v + i), vb = ldg2(it.v + i1);
                         const float2 a = xform(mq, va.x, va.y), b = xform(mq, vb.x, vb.y);
                         gm = make_float4(a.x, a.y, b.x, b.y);
-                        root = (uint32_t)L.vroot[qi];
+                        const uint32_t vr = L.vroot[qi];
+                        start[0] = vr & ~VR_COLLECTS;
                         // the candidates this edge's box may collect (all of them when the
                         // query has more than NC); an edge whose candidates are all in the
                         // set already adds nothing
@@ -589,10 +560,16 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                             }
                         }
                         want = (em & ~L.cdone[qi]) != 0u;
-                        const uint32_t vc = L.vcell[qi];
-                        if (want && !(vc & VR_COLLECTS))
-                            root = collect_start_cells(c, entity_box(false, gm), root, L.vdepth[qi], L.vbox[qi],
-                                                       vc & 0xffffu, (vc >> 16) & 0x7fffu);
+                        if (want && !(vr & VR_COLLECTS)) {
+                            const EdgeCells ec = edge_cells(c.grid, c.cell_level, root_bb, entity_box(false, gm));
+                            if (ec.l > L.vdepth[qi]) {
+                                start[0] = collect_start(c, ec.l, ec.x0, ec.y0);
+                                if (ec.x0 != ec.x1 || ec.y0 != ec.y1) {
+                                    start[1] = collect_start(c, ec.l, ec.x1, ec.y1);
+                                    more[1] = start[1] != start[0];
+                                }
+                            }
+                        }
                     }
                 }
             }
@@ -606,7 +583,13 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                 L.geom[o] = gm;
                 L.emask[o] = em;
                 L.ent_slot[o] = (uint8_t)(qi | (circle ? WL_CIRCLE : 0u));
-                L.nodes[o] = (o << 24) | root;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; j++) {
+                const bool put = want && rank < room && more[j];
+                const uint64_t pb = __ballot(put);
+                if (put) L.nodes[nn + lanes_below(pb, lane)] = ((n + rank) << 24) | start[j];
+                nn += (uint32_t)__builtin_popcountll(pb);
             }
             if (n_want <= room) {
                 n += n_want;
@@ -619,7 +602,7 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                 n = CL_ENT;
             }
         }
-        wave_collect(c, L, n, lane);
+        wave_collect(c, L, nn, lane);
     }
     // containment over the virtual root's Partial hazards not yet collected
     // (cd_engine.rs:276-287), by the query's CG lanes: a candidate without bbox relation
@@ -664,7 +647,9 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
     if (active) {
         const uint32_t* t = L.set + qs * SET_CAP;
         if (L.ovf[qs]) {
-            if (sub == 0) {
+            if (DIRECT) {
+                if (sub == 0) count[out] = COUNT_OVERFLOW;
+            } else if (sub == 0) {
                 const uint32_t at = atomicAdd(&counters[C_OVERFLOW], 1u);
                 ovf[at] = ((uint64_t)set_index << 32) | (uint32_t)(q0 + qs);
             }
@@ -713,14 +698,46 @@ __global__ __launch_bounds__(WAVE, CL_WAVES) void k_collect_units(const SetDesc*
         const uint32_t si = wave_bcast(un.set);
         for (uint32_t p0 = 0; p0 < un.count; p0 += CP) {
             const uint32_t P = un.count - p0 < CP ? un.count - p0 : CP;
-            collect_pass(sets[si], si, un.q0 + p0, P, lds, m6, cap, count, hash, keys, counters, ovf, lane);
+            collect_pass<false>(sets[si], si, un.q0 + p0, P, lds, m6, cap, count, hash, keys, counters, ovf, lane);
         }
+    }
+}
+
+// One set without a table, for jg_collect_batch: the descriptor comes by value, workgroup b collects
+// the `chunk` <= CP queries from b * chunk on (then every gridDim.x-th such pass).
+__global__ __launch_bounds__(WAVE, CL_WAVES) void k_collect_direct(SetDesc sd, uint32_t n, uint32_t chunk,
+                                                                   const float* __restrict__ m6, uint32_t cap,
+                                                                   uint32_t* __restrict__ count, uint64_t* __restrict__ hash,
+                                                                   uint32_t* __restrict__ keys) {
+    __shared__ CollectLds lds;
+    const uint32_t n_passes = (n - 1u) / chunk + 1u;
+    for (uint32_t u = blockIdx.x; u < n_passes; u += gridDim.x) {
+        const uint32_t q0 = u * chunk;
+        collect_pass<true>(sd, 0u, q0, n - q0 < chunk ? n - q0 : chunk, lds, m6, cap, count, hash, keys, nullptr, nullptr,
+                           threadIdx.x);
     }
 }
 
 }  // namespace
 
 namespace jg {
+
+jg_status collect_direct_launch(const CdeView& cde, const ItemView& item, const float* d_m6, uint64_t n, uint32_t cap,
+                                uint32_t* d_count, uint64_t* d_hash, uint32_t* d_keys, uint32_t n_cus, hipStream_t stream) {
+    SetDesc sd{};
+    sd.cde = cde;
+    sd.item = item;
+    // Queries per wave: as few as keep the launch within the waves that run at once, since a wave's
+    // time grows with its queries.  us at 1 / 2 / 4 / 8 (64-vertex item, 2000-item sheet): 64 queries
+    // 47 / 49 / 78 / 138, 4096 73 / 104 / 120 / 185, 10000 121 / 108 / 124 / 190, 200000 1318 / 998 /
+    // 930 / 939 (one query per wave with the bitmask collector, k_collect: 69, 96, 198, 2557).
+    uint32_t chunk = 1;
+    while (chunk < CP && (n + chunk - 1) / chunk > (uint64_t)n_cus * 4u * CL_WAVES) chunk <<= 1;
+    const uint64_t passes = (n + chunk - 1) / chunk;
+    hipLaunchKernelGGL(k_collect_direct, dim3((uint32_t)std::min<uint64_t>(passes, 1u << 20)), dim3(WAVE), 0, stream, sd,
+                       (uint32_t)n, chunk, d_m6, cap, d_count, d_hash, d_keys);
+    return hip_check(hipGetLastError(), "collect launch");
+}
 
 jg_status collect_launch(const TableLayout& L, uint8_t* base, const float* d_m6, uint32_t cap, uint32_t* d_count,
                          uint64_t* d_hash, uint32_t* d_keys, uint64_t* ovf, uint32_t n_cus, hipStream_t stream) {

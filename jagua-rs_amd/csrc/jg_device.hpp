@@ -204,23 +204,6 @@ __device__ __forceinline__ int virtual_root(const CdeView& c, float4 bb) {
     return virtual_root(c, bb, depth);
 }
 
-// The cell (ix, iy) at level `depth` of a node whose box `box` is a quadrant `depth` levels below
-// the root box: the quadrants holding the box's centre (strictly on one side of every midline
-// above it, as the box is one of the subdivision's).
-__device__ __forceinline__ void node_cell(float4 root, float4 box, uint32_t depth, uint32_t& ix, uint32_t& iy) {
-    const float cx = (box.x + box.z) / 2.0f, cy = (box.y + box.w) / 2.0f;
-    float4 r = root;
-    ix = 0;
-    iy = 0;
-    for (uint32_t l = 0; l < depth; l++) {
-        const float mxm = (r.x + r.z) / 2.0f, mym = (r.y + r.w) / 2.0f;
-        const bool xh = cx > mxm, yh = cy > mym;
-        r = make_float4(xh ? mxm : r.x, yh ? mym : r.y, xh ? r.z : mxm, yh ? r.w : mym);
-        ix = 2u * ix + (xh ? 1u : 0u);
-        iy = 2u * iy + (yh ? 1u : 0u);
-    }
-}
-
 __device__ __forceinline__ uint32_t cell_entry(const CdeView& c, uint32_t l, uint32_t ix, uint32_t iy) {
     return ldg1(c.cells + ((1u << (2u * l)) - 1u) / 3u + ((iy << l) | ix));
 }

@@ -38,6 +38,26 @@ def test_detect_sizes(cuda, sheet, n, filt):
     assert (got[n:] == 99).all(), "written past the batch"
 
 
+@pytest.mark.parametrize("n,nv,r", [(1, 40, 20.0), (5 * CUS16 // 4, 40, 20.0), (5 * CUS16 // 4 + 1, 12, 20.0),
+                                    (40 * CUS16 // 4 + 3, 9, 15.0), (130, 24, 400.0)])
+def test_collect_sizes(cuda, sheet, n, nv, r):
+    """The last item covers more hazards than a query's collector holds (16): those queries are
+    collected by the second launch."""
+    cde, keys, oc, cont = sheet
+    (item,), (oitem,) = items([S.polygon(76, nv, nv, 0.5 * r, r, 2)])
+    mats = J.compose(S.transforms(77 + n, n, (0.0, 0.0, float(cont[:, 0].max()), float(cont[:, 1].max())), 0))
+    out = (torch.full((n + 8,), -7, dtype=torch.int32, device=cuda), torch.full((n + 8,), -7, dtype=torch.int64, device=cuda),
+           torch.full((n + 8, 20), -7, dtype=torch.int32, device=cuda))
+    cde.collect_batch(item, torch.from_numpy(mats).to(cuda), capacity=20, out=tuple(t[:n] for t in out))
+    ref = O.query(oc, oitem, mats=mats, mode=3, keys_cap=20, threads=8)
+    got = [t.cpu().numpy() for t in out]
+    np.testing.assert_array_equal(got[0][:n].astype(np.uint32), ref["count"])
+    np.testing.assert_array_equal(got[1][:n].view(np.uint64), ref["hash"])
+    np.testing.assert_array_equal(got[2][:n].view(np.uint32), ref["keys"])
+    assert all((g[n:] == -7).all() for g in got), "written past the batch"
+    assert r < 100.0 or (ref["count"] > 16).sum() > 20
+
+
 def test_detect_captured(cuda, sheet):
     """One call captured and replayed on new transforms in the same buffer."""
     cde, keys, oc, cont = sheet
