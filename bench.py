@@ -220,7 +220,7 @@ def run_c2(args):
         graph_ok = bool(torch.equal(status_graph, status))
         # hazard sets of the same step (collect_surrogate_collisions U collect_poly_collisions,
         # ci_bench.rs:56-69): count, hash and the first 8 keys per query, all sets in one
-        # persistent launch; the per-query kernel (one launch per item) beside it
+        # launch; one collect_batch per item beside it
         plan.collect(mats_all, capacity=cap, count=cnt, hash=hsh, keys=keys)
         ms_collect = timed(lambda: plan.collect(mats_all, capacity=cap, count=cnt, hash=hsh, keys=keys),
                            args.steps, stream)
@@ -237,7 +237,7 @@ def run_c2(args):
         ms_collect_plain = timed(collect_plain_step, 2, stream)
         collect_forms_agree = bool(torch.equal(cnt, cnt_p) and torch.equal(hsh, hsh_p) and torch.equal(keys, keys_p))
         log(f"collect: batched {ms_collect:.3f} ms/step ({total / (ms_collect / 1e3) / 1e6:.1f} M queries/s), "
-            f"per-query kernel {ms_collect_plain:.3f} ms; same sets: {collect_forms_agree}")
+            f"one launch per item {ms_collect_plain:.3f} ms; same sets: {collect_forms_agree}")
         result["forms"] = {
             "plain_queries_per_s": total / (ms_plain_wave / 1e3), "plain_ms_per_step": ms_plain_wave,
             "plain_form": f"the batched kernels, one plan per (layout, item) set, {len(items)} plans launched "
@@ -257,7 +257,7 @@ def run_c2(args):
             result["forms"]["collect_profile"] = {
                 "bound": cprof.get("bound"), "traffic": cprof.get("traffic"), "lane_util": ck["lane_util"],
                 "valu_issue": ck["valu_issue"], "wait_share": ck["wait_share"], "file": "profiles/pmc_collect_config2.md"}
-        log(f"plain (per-set plans) {ms_plain_wave:.3f} ms/step, scalar {ms_scalar:.3f} ms, graph {ms_graph:.3f} ms; "
+        log(f"plain (per-set plans) {ms_plain_wave:.3f} ms/step, one launch per item {ms_scalar:.3f} ms, graph {ms_graph:.3f} ms; "
             f"same verdicts: {plain_wave_ok and scalar_ok and graph_ok}")
         result["overlap"] = overlap_c4(stream)
         result["search"] = search_c2(cde, items, stream)

@@ -620,12 +620,59 @@ FilterView set_filter(const jg_query_set& s, const jg_hazard_filter& f, const ui
     return v;
 }
 
+// Lanes per query and queries per unit where the schedule leaves them open.  `compact`: the forms
+// whose tables bound what jg_detect_sets_noalloc takes.
+uint32_t table_lanes(const jg_plan_config& cfg, uint32_t v, uint64_t n_all, uint32_t n_cus, bool compact) {
+    uint32_t lanes = cfg.lanes_per_query;
+    if (lanes == 0 && compact) {
+        lanes = 8;
+        while (lanes < v && lanes < 32u) lanes <<= 1;
+    } else if (lanes == 0) {
+        // by vertices in a large launch: us per step at up to 32 lanes (the vertices rounded up) / at
+        // these / at 64 for all above 32, 552 / 539 / 592 (2000-item sheet), 363 / 333 / 345
+        // (concave items of 300 vertices at the mean).  A launch with waves to spare, a query
+        // or less for each after the surrogate stage: the whole wave, as its time is a pass's
+        // (32000 queries of 64 items of 8-512 vertices: 93 -> 81 us).
+        lanes = v <= 16u ? 8u : v <= 64u ? 16u : v <= 384u ? 32u : 64u;
+        if (n_all <= (uint64_t)n_cus * 160u) lanes = 64u;
+    }
+    uint32_t pow2 = 1;
+    while (pow2 < lanes && pow2 < 64u) pow2 <<= 1;
+    return pow2;
+}
+
+uint32_t table_chunk(const jg_plan_config& cfg, uint64_t n_all, uint32_t n_cus, bool compact) {
+    // 16, 32 or 64; 64 packs 128 pole entities into one surrogate traversal; smaller units shorten the
+    // fused kernel's tail (32 by default in a launch with waves to spare: 16000 queries of
+    // 64-vertex items 63 -> 55 us)
+    if (cfg.chunk == 0) return !compact && n_all <= (uint64_t)n_cus * 160u ? 32u : 64u;
+    return cfg.chunk <= 16u ? 16u : cfg.chunk <= 32u ? 32u : 64u;
+}
+
+// What the sets' compact table counts against JG_NOALLOC_SCRATCH_BYTES, whatever the schedule's
+// defaults choose: descriptors, units, COMPACT_FIXED bytes of counters and bases, groups.
+constexpr size_t COMPACT_FIXED = 3360;
+uint64_t compact_table_bytes(const std::vector<jg_query_set>& sets, const jg_plan_config& cfg) {
+    const uint32_t uq = table_chunk(cfg, 0, 0, true);
+    uint64_t units = 0, groups = 0;
+    for (auto& s : sets) {
+        const uint32_t per = 64u / table_lanes(cfg, s.item->poly.n(), 0, 0, true);
+        const uint64_t full = s.count / uq, rest = s.count % uq;
+        units += full + (rest ? 1u : 0u);
+        groups += full * ((uq + per - 1u) / per) + (rest + per - 1u) / per;
+    }
+    const uint64_t o_units = (sizeof(SetDesc) * sets.size() + 255) & ~255ull;
+    const uint64_t o_ctr = (o_units + sizeof(Unit) * units + 255) & ~255ull;
+    return ((o_ctr + COMPACT_FIXED + 255) & ~255ull) + sizeof(Group) * (groups + 1);
+}
+
 // The host bytes of the table of `sets` under schedule `cfg`, given each set's item view and
 // filter view (device addresses), and its layout.
 // seeds[i] (device address, count): the slots set i's collectors start with (may be empty).
 jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<ItemView>& iv,
                       const std::vector<FilterView>& fv, const std::vector<std::pair<const uint32_t*, uint32_t>>& seeds,
-                      const jg_plan_config& cfg, uint32_t n_cus, std::vector<uint8_t>& host, TableLayout& L) {
+                      const jg_plan_config& cfg, uint32_t n_cus, std::vector<uint8_t>& host, TableLayout& L,
+                      bool compact = false) {
     for (auto& s : sets) {
         if (s.cde->view.n_nodes >= WL_MAX_NODES)
             return fail(JG_ERR_CAPACITY, "quadtree of more than 2^24 nodes in a batched plan");
@@ -652,20 +699,7 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
         sd[i].flags = cfg.flags ? cfg.flags : (JG_QUERY_SURROGATE | JG_QUERY_POLY);
         if (!(sd[i].flags & JG_QUERY_SURROGATE)) { sd[i].item.n_poles = 0; sd[i].item.n_piers = 0; }
         sd[i].first = s.first;
-        uint32_t lanes = cfg.lanes_per_query;
-        if (lanes == 0) {
-            // by vertices in a large launch: us per step at up to 32 lanes (the vertices rounded up) / at
-            // these / at 64 for all above 32, 552 / 539 / 592 (2000-item sheet), 363 / 333 / 345
-            // (concave items of 300 vertices at the mean).  A launch with waves to spare, a query
-            // or less for each after the surrogate stage: the whole wave, as its time is a pass's
-            // (32000 queries of 64 items of 8-512 vertices: 93 -> 81 us).
-            const uint32_t v = s.item->poly.n();
-            lanes = v <= 16u ? 8u : v <= 64u ? 16u : v <= 384u ? 32u : 64u;
-            if (n_all <= (uint64_t)n_cus * 160u) lanes = 64u;
-        }
-        uint32_t pow2 = 1;
-        while (pow2 < lanes && pow2 < 64u) pow2 <<= 1;
-        sd[i].lanes = pow2;
+        sd[i].lanes = table_lanes(cfg, s.item->poly.n(), n_all, n_cus, compact);
         sd[i].filter = fv[i];
         any_filter = any_filter || sd[i].filter.kind != 0;
         any_pole = any_pole || sd[i].item.n_poles > 0;
@@ -674,11 +708,8 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
     L.filtered = any_filter;
     L.kind = any_pier ? (any_pole ? KIND_MIXED : KIND_EDGE) : KIND_CIRCLE;
     L.stages = cfg.stages == 1u ? 1u : 2u;
-    // work units: sets in decreasing item size, `chunk` queries each (16, 32 or 64; 64 packs
-    // 128 pole entities into one surrogate traversal; smaller units shorten the fused kernel's
-    // tail)
-    // (32 by default in a launch with waves to spare: 16000 queries of 64-vertex items 63 -> 55 us)
-    const uint32_t uq = cfg.chunk == 0 ? (n_all <= (uint64_t)n_cus * 160u ? 32u : 64u) : cfg.chunk <= 16u ? 16u : cfg.chunk <= 32u ? 32u : 64u;
+    // work units: sets in decreasing item size, `chunk` queries each
+    const uint32_t uq = table_chunk(cfg, n_all, n_cus, compact);
     std::vector<size_t> order(sets.size());
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
@@ -705,6 +736,7 @@ jg_status table_image(const std::vector<jg_query_set>& sets, const std::vector<I
     for (uint32_t x = 0; x < N_STREAMS; x++) {
         gbase[x] = (uint32_t)max_groups;
         max_groups += stream_groups[x];
+        if (max_groups >= 0xffffffffull && !compact) return table_image(sets, iv, fv, seeds, cfg, n_cus, host, L, true);
         if (max_groups >= 0xffffffffull) return fail(JG_ERR_CAPACITY, "too many survivor groups in a batched plan");
     }
     L.o_grp = (L.o_gbase + sizeof(gbase) + 255) & ~(size_t)255;
@@ -968,7 +1000,10 @@ extern "C" jg_status jg_plan_detect_graph(jg_plan* p, const float* d_m6, uint8_t
 // device array of JG_NOALLOC_SCRATCH_BYTES that every call on a device shares.  Host code
 // never passes the array's name to the device: `scratch` names a host-side shadow, and its
 // device address comes from hipGetSymbolAddress, once per device.
-static __device__ __align__(256) uint8_t scratch[JG_NOALLOC_SCRATCH_BYTES];
+// SCRATCH_EXTRA holds what a table's counters take over COMPACT_FIXED.
+constexpr size_t SCRATCH_EXTRA = 8192;
+static_assert(4u * (N_COUNTER_WORDS + N_STREAMS) + 255u <= COMPACT_FIXED + SCRATCH_EXTRA, "extra scratch must cover the counters");
+static __device__ __align__(256) uint8_t scratch[JG_NOALLOC_SCRATCH_BYTES + SCRATCH_EXTRA];
 
 namespace {
 constexpr int MAX_DEVICES = 64;
@@ -1062,11 +1097,16 @@ extern "C" jg_status jg_detect_sets_noalloc(const jg_query_set* sets, uint32_t n
     TableLayout L;
     st = table_image(vs, iv, fv, {}, pc, cus, table, L);
     if (st != JG_OK) return st;
-    const uint64_t need = (uint64_t)o_table + L.total;
+    const uint64_t need = (uint64_t)o_table + compact_table_bytes(vs, pc);
     if (need > JG_NOALLOC_SCRATCH_BYTES)
         return fail(JG_ERR_CAPACITY, "jg_detect_sets_noalloc needs " + std::to_string(need) +
                                          " bytes of scratch; the fixed scratch holds " +
                                          std::to_string((uint64_t)JG_NOALLOC_SCRATCH_BYTES));
+    if (o_table + L.total > sizeof(scratch)) {
+        st = table_image(vs, iv, fv, {}, pc, cus, table, L, true);
+        if (st != JG_OK) return st;
+        if (o_table + L.total > sizeof(scratch)) return fail(JG_ERR_INTERNAL, "compact table past the scratch");
+    }
     host.resize(o_table + table.size());
     std::memcpy(host.data() + o_table, table.data(), table.size());
     // pageable source: the copy is complete when the call returns, and ordered on `stream`

@@ -302,7 +302,7 @@ __device__ __forceinline__ bool collides_edge(const CdeView& c, int start, float
 // Wave-cooperative traversal.  QTNode::collides (qt_node.rs:99-147) answers whether any
 // relevant hazard of the subtree collides with the entity; its recursion order only decides
 // which hazard is found first.  A wave therefore turns all descents of its entities (up to
-// WL_ENT circles or edges, each belonging to one query slot) into two LDS queues: node visits
+// ENT circles or edges, each belonging to one query slot) into two LDS queues: node visits
 // (entity, node) and edge tests (entity, hazard edge).  Each step takes 64 items of one kind:
 //   node step: the visit's strongest relevant hazard (qt_hazard_vec.rs:60-63) is Entire -> hit;
 //              an internal node pushes the colliding quadrants (qt_traits.rs); a leaf pushes one

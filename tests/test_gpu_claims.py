@@ -43,3 +43,22 @@ def test_every_item_is_taken(cuda, layout, n, workgroups, stages):
             cnt, hsh, _ = plan.collect(m, capacity=0)
             np.testing.assert_array_equal(cnt.cpu().numpy().astype(np.uint32), np.concatenate([r["count"] for r in ref]))
             np.testing.assert_array_equal(hsh.cpu().numpy().view(np.uint64), np.concatenate([r["hash"] for r in ref]))
+
+
+@pytest.mark.parametrize("item", [1, 2])
+def test_noalloc_takes_what_its_scratch_was_sized_for(cuda, layout, item):
+    """33 B of table per 4 queries (a unit per 64, a group per 2), whatever lanes the default
+    schedule would give the item: about 4.066 million queries fit 32 MiB."""
+    cde, oc, prod, orc, box = layout
+    cde.sync()
+    base = J.compose(S.transforms(97, 40000, box, 0))
+    n = 4_064_000
+    m = torch.from_numpy(base).to(cuda).repeat(n // 40000 + 1, 1)[:4_069_000].contiguous()
+    out = torch.full((4_069_000,), 99, dtype=torch.uint8, device=cuda)
+    with pytest.raises(J.JaguaError, match="scratch"):
+        J.detect_sets_noalloc([(cde, prod[item], 0, 4_069_000, None)], m, out)
+    J.detect_sets_noalloc([(cde, prod[item], 0, n, None)], m, out)
+    ref = O.query(oc, orc[item], mats=base, mode=1, threads=8)["status"]
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:n], np.tile(ref, n // 40000 + 1)[:n])
+    assert (got[n:] == 99).all()
