@@ -334,7 +334,8 @@ JG_HD HoldingCell holding_cell(const CellGrid& g, uint32_t level, float4 root, f
 //  - below it, the edge leaves the node across that side only; its endpoint lies strictly inside the
 //    quadrant on the path, and the other three are disjoint, beyond the endpoint or the midline.
 // "Strictly" is by the margin of holding_cell, for the endpoints against the crossed side as well;
-// where it fails, one cell of a level above is taken.
+// where it fails, one cell of a level above is taken.  An edge with a NaN lies inside no quadrant:
+// l = 0, no cell below the node that its descent starts from.
 struct EdgeCells {
     uint32_t l, x0, y0, x1, y1;
 };
@@ -343,9 +344,10 @@ JG_HD EdgeCells edge_cells(const CellGrid& g, uint32_t level, float4 root, float
     const uint32_t x0 = grid_index(b.x - g.eps - root.x, g.sx, top), x1 = grid_index(b.z + g.eps - root.x, g.sx, top);
     const uint32_t y0 = grid_index(b.y - g.eps - root.y, g.sy, top), y1 = grid_index(b.w + g.eps - root.y, g.sy, top);
     const uint32_t d = (x0 ^ x1) | (y0 ^ y1);
-    uint32_t s = !(g.sx > 0.0f) ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
+    const bool ok = g.sx > 0.0f && b.x <= b.z && b.y <= b.w;
+    uint32_t s = !ok ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
     EdgeCells o{level - s, x0 >> s, y0 >> s, x0 >> s, y0 >> s};
-    if (s != 0u && g.sx > 0.0f) {
+    if (s != 0u && ok) {
         const uint32_t x2 = grid_index(b.x + g.eps - root.x, g.sx, top), x3 = grid_index(b.z - g.eps - root.x, g.sx, top);
         const uint32_t y2 = grid_index(b.y + g.eps - root.y, g.sy, top), y3 = grid_index(b.w - g.eps - root.y, g.sy, top);
         uint32_t t = 0;                       // the least shift with at most two cells, side by side

@@ -6,6 +6,7 @@
 // bounds and a few ulps beside them; edges likewise inside it.
 // Usage: start_cells_check <seed> <cases>; prints "ok <leaves> <on bounds> <edges with two cells>".
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -186,6 +187,14 @@ int main(int argc, char** argv) {
                 return 1;
             }
             // the virtual root's path: the quadrant that surrounds the box, as the search takes it
+            // an edge of NaNs has no cell of its own, and a box that is empty along an axis no holding cell
+            const float4 en = make_float4(q & 1 ? NAN : eb.x, q & 2 || !(q & 1) ? NAN : eb.y, q & 1 ? NAN : eb.z, q & 2 || !(q & 1) ? NAN : eb.w);
+            const float4 bn = make_float4(en.x == en.x ? en.x : FLT_MAX, en.y == en.y ? en.y : FLT_MAX,
+                                          en.z == en.z ? en.z : -FLT_MAX, en.w == en.w ? en.w : -FLT_MAX);
+            if (edge_cells(g, t.table, t.root, en).l != 0u || holding_cell(g, t.table, t.root, bn).l != 0u) {
+                std::printf("a NaN edge or an empty box has a cell\n");
+                return 1;
+            }
             uint32_t d, x, y;
             deepest(t, hc.l, hc.ix, hc.iy, d, x, y);
             uint32_t rx = 0, ry = 0;
