@@ -511,8 +511,8 @@ __global__ __launch_bounds__(WAVE, 4) void k_fused_filtered(const SetDesc* __res
 // Nothing is allocated, claimed or left behind, so calls on any streams and threads, captured or
 // not, are independent.  A small batch is bound by the latency of one query's descent, so its
 // queries are spread over as many waves as the chip runs: 64 queries against a 40-item strip
-// take 18 us, 5000 against a 2000-item sheet 42 us; one query per lane, each descending by
-// itself, took 183 and 1227.
+// take 17 us, 5000 against a 2000-item sheet 33 us; one query per lane, each descending by
+// itself, took 206 and 947.
 template <bool FILT, int KIND>
 __global__ __launch_bounds__(WAVE, 4) void k_detect_direct(SetDesc sd, uint32_t n, uint32_t chunk,
                                                            const float* __restrict__ m6, uint8_t* __restrict__ status) {
@@ -554,14 +554,18 @@ jg_status detect_direct_launch(const CdeView& cde, const ItemView& item, const F
     sd.filter = filter;
     sd.flags = flags;
     // Queries per wave: one while the chip has waves to spare (16 per compute unit), then as few as
-    // keep the launch within that many, up to 16.  A wave's time grows with its queries long
-    // before its lanes are full, so small batches are quickest spread out; beyond 16 a unit's
-    // polygon stage is the tail.  Measured on a 2000-item layout (64-vertex item), us at 1 / 2 / 4 /
-    // 16 / 64 queries per wave: 1000 queries 28 / 29 / 32 / 41 / 115, 5000 44 / 42 / 43 / 55 / 137,
-    // 16384 70 / 52 / 45 / 56 / 135, 65536 211 / 130 / 89 / 72 / 146, 262144 781 / 452 / 282 / 179 / 189.
+    // keep the launch within that many, up to 16, as a wave's time grows with its queries long
+    // before its lanes are full; 32 and 64, which fill them, once the launch is three times that deep
+    // at 16 and at 32, but for filtered queries of large items, whose polygon stages then make the
+    // tail (300 vertices, 500000 queries: 549 us at 16, 600 at 32; without a filter 297 and 222).
+    // us at 1 / 2 / 4 / 16 / 32 / 64 queries per wave (2000-item layout, 64-vertex item):
+    // 1000 queries 18 / 20 / 21 / 26 / 32 / 41, 5000 34 / 35 / 34 / 39 / 47 / 62, 16384 49 / 40 / 36 / 41 / 49 /
+    // 61, 65536 154 / 100 / 76 / 73 / 77 / 101, 262144 548 / 338 / 217 / 130 / 114 / 108,
+    // 1000000 (16 on) 385 / 260 / 221.
     const uint64_t waves = (uint64_t)device_cus() * 16u;
     uint32_t chunk = 1;
-    while (chunk < 16u && (n + chunk - 1) / chunk > waves) chunk <<= 1;
+    const uint32_t most = filter.kind == 0u || item.n_v <= 64u ? 64u : 16u;
+    while (chunk < most && (n + chunk - 1) / chunk > (chunk < 16u ? waves : 3u * waves)) chunk <<= 1;
     // lanes per query in the polygon stage: the plan's rule, and at least the wave over its queries
     uint32_t lanes = 8;
     while (lanes < item.n_v && lanes < 32u) lanes <<= 1;

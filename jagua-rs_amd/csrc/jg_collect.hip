@@ -729,8 +729,8 @@ jg_status collect_direct_launch(const CdeView& cde, const ItemView& item, const 
     sd.item = item;
     // Queries per wave: as few as keep the launch within the waves that run at once, since a wave's
     // time grows with its queries.  us at 1 / 2 / 4 / 8 (64-vertex item, 2000-item sheet): 64 queries
-    // 47 / 49 / 78 / 138, 4096 73 / 104 / 120 / 185, 10000 121 / 108 / 124 / 190, 200000 1318 / 998 /
-    // 930 / 939 (one query per wave with the bitmask collector, k_collect: 69, 96, 198, 2557).
+    // 41 / 49 / 67 / 123, 4096 62 / 63 / 92 / 147, 10000 118 / 86 / 116 / 158, 200000 1257 / 954 /
+    // 866 / 853 (one query per wave with the bitmask collector, k_collect: 69, 96, 198, 2557).
     uint32_t chunk = 1;
     while (chunk < CP && (n + chunk - 1) / chunk > (uint64_t)n_cus * 4u * CL_WAVES) chunk <<= 1;
     const uint64_t passes = (n + chunk - 1) / chunk;

@@ -38,6 +38,21 @@ def test_detect_sizes(cuda, sheet, n, filt):
     assert (got[n:] == 99).all(), "written past the batch"
 
 
+@pytest.mark.parametrize("n,nv,filt", [(48 * CUS16, 24, False), (48 * CUS16 + 1, 24, True), (96 * CUS16 + 1, 64, True),
+                                       (96 * CUS16 + 1, 65, False), (96 * CUS16 + 1, 65, True)])
+def test_detect_full_waves(cuda, sheet, n, nv, filt):
+    """16, 32 and 64 queries per wave; 16 at most for filtered queries of more than 64 vertices."""
+    cde, keys, oc, cont = sheet
+    (item,), (oitem,) = items([S.polygon(78, nv, nv, 10.0, 30.0, 2)])
+    mats = J.compose(S.transforms(79, n, (0.0, 0.0, float(cont[:, 0].max()), float(cont[:, 1].max())), 0))
+    out = torch.full((n + 8,), 99, dtype=torch.uint8, device=cuda)
+    cde.detect_batch(item, torch.from_numpy(mats).to(cuda), J.HashedFilter(5, 0.1) if filt else None, out=out[:n])
+    ref = O.query(oc, oitem, mats=mats, mode=1, filt=O.make_filter(2, 5, J.HashedFilter(5, 0.1).threshold) if filt else None, threads=8)
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:n], ref["status"])
+    assert (got[n:] == 99).all()
+
+
 @pytest.mark.parametrize("n,nv,r", [(1, 40, 20.0), (5 * CUS16 // 4, 40, 20.0), (5 * CUS16 // 4 + 1, 12, 20.0),
                                     (40 * CUS16 // 4 + 3, 9, 15.0), (130, 24, 400.0)])
 def test_collect_sizes(cuda, sheet, n, nv, r):
