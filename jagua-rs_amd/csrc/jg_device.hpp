@@ -211,7 +211,7 @@ __device__ __forceinline__ uint32_t cell_entry(const CdeView& c, uint32_t l, uin
 // virtual_root through the cell tables: at every level above the cell that strictly holds bb, that
 // cell's quadrant is the one that surrounds bb, so the search passes the deepest node on the path
 // to it; it ends there if that node lies above the cell's level, and goes on through node records
-// otherwise.  bb lies within the root box.
+// otherwise.
 __device__ __forceinline__ int virtual_root_cells(const CdeView& c, float4 root, float4 bb, uint32_t& depth) {
     const HoldingCell h = holding_cell(c.grid, c.cell_level, root, bb);
     const uint32_t e = cell_entry(c, h.l, h.ix, h.iy);

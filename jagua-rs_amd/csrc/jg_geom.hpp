@@ -303,7 +303,8 @@ JG_HD CircleCells circle_cells(const CellGrid& g, uint32_t level, float4 root, f
 // The cell that strictly holds a box: (ix, iy) of level l, the deepest of the even grid's cells that
 // the box, widened by the grid's margin, lies in.  A cell's bounds as the tree builds them,
 // midpoints of midpoints, are a few ulps off the even grid, so the box lies strictly on one side
-// of every midline above the cell.  (l = 0 without a grid.)
+// of every midline above the cell.  (l = 0 without a grid, and for a box that leaves the root box,
+// which no quadrant surrounds.)
 struct HoldingCell {
     uint32_t l, ix, iy;
 };
@@ -312,7 +313,8 @@ JG_HD HoldingCell holding_cell(const CellGrid& g, uint32_t level, float4 root, f
     const uint32_t x0 = grid_index(b.x - g.eps - root.x, g.sx, top), x1 = grid_index(b.z + g.eps - root.x, g.sx, top);
     const uint32_t y0 = grid_index(b.y - g.eps - root.y, g.sy, top), y1 = grid_index(b.w + g.eps - root.y, g.sy, top);
     const uint32_t d = (x0 ^ x1) | (y0 ^ y1);
-    const uint32_t s = !(g.sx > 0.0f) ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
+    const bool ok = g.sx > 0.0f && b.x >= root.x && b.y >= root.y && b.z <= root.z && b.w <= root.w;
+    const uint32_t s = !ok ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
     return HoldingCell{level - s, x0 >> s, y0 >> s};
 }
 
