@@ -348,8 +348,7 @@ __device__ __forceinline__ void poly_queries(const SetDesc& sd, uint32_t q0, uin
                     gm[j] = make_float4(a.x, a.y, b2.x, b2.y);
                     W.geom[o] = gm[j];
                     W.ent_slot[o] = (uint8_t)slot;
-                    const float4 eb = make_float4(mn(a.x, b2.x), mn(a.y, b2.y), mx(a.x, b2.x), mx(a.y, b2.y));
-                    edge_starts(c, root_bb, vr_depth, eb, n0[j], n1[j]);
+                    edge_starts(c, root_bb, vr_depth, gm[j], n0[j], n1[j]);
                 }
             }
 #pragma unroll

@@ -68,7 +68,9 @@ constexpr uint32_t SURR_MASK = 0u;       // emask of a pole or pier: the node-en
 constexpr uint32_t C_EXT = 0x80000000u;  // candidate record flags: exterior hazard, Entire in the virtual root
 constexpr uint32_t C_ENTIRE = 0x40000000u;
 constexpr uint32_t C_SLOT = 0x3fffffffu;
-constexpr uint32_t VR_COLLECTS = 0x80000000u;   // vroot flag: the virtual root collects
+constexpr uint32_t VR_COLLECTS = 0x80000000u;   // vroot flags: the virtual root collects; the query's bbox
+constexpr uint32_t VR_INSIDE = 0x40000000u;     // lies inside the root box
+constexpr uint32_t VR_NODE = WL_NODE_MASK;
 
 struct CollectLds {
     uint32_t nodes[CL_NCAP];             // entity << 24 | node
@@ -83,7 +85,7 @@ struct CollectLds {
     uint32_t cdone[CP];                  // bit i: candidate i is in the set
     uint32_t ovf[CP];                    // per query: its set outgrew SET_CAP
     uint32_t vroot[CP];                  // the virtual root | VR_COLLECTS when it collects (a leaf, or at
-                                         // most cd_threshold active edges)
+                                         // most cd_threshold active edges) | VR_INSIDE
     uint32_t vdepth[CP];                 // its depth
     float mat[CP][6];                    // per query: its transformation
     float4 qbox[CP];                     // per query: its transformed bbox
@@ -428,6 +430,7 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
         ve0 = vn.haz_begin;
         vcnt = vn.haz_info & COUNT_MASK;
         vcoll = (vn.first_child < 0 || vn.n_active_edges <= c.cd_threshold) ? VR_COLLECTS : 0u;
+        vcoll |= box_relation(root_bb, bb) == REL_SURROUNDING ? VR_INSIDE : 0u;
     }
     if (sub == 0) {
         L.vroot[qs] = (uint32_t)vr | vcoll;
@@ -488,7 +491,7 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
         // a pre-seeded collector, then the exterior when the shape leaves the engine's bbox
         // (cd_engine.rs:262-264); the traversal goes on regardless
         for (uint32_t i = sub; i < sd.n_seed; i += CG) set_put(L, qs, ldg1(sd.seed + i));
-        if (sub == 0 && box_relation(ldg4((const float4*)c.nodes), bb) != REL_SURROUNDING) set_put(L, qs, c.exterior_slot);
+        if (sub == 0 && !(L.vroot[qs] & VR_INSIDE)) set_put(L, qs, c.exterior_slot);
     }
     // every query's ff poles / piers from the root and edges from its virtual root.  A cursor
     // walks the entities 64 at a time; those that may add to their query's set take the next
@@ -542,7 +545,7 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                         const float2 a = xform(mq, va.x, va.y), b = xform(mq, vb.x, vb.y);
                         gm = make_float4(a.x, a.y, b.x, b.y);
                         const uint32_t vr = L.vroot[qi];
-                        start[0] = vr & ~VR_COLLECTS;
+                        start[0] = vr & VR_NODE;
                         // the candidates this edge's box may collect (all of them when the
                         // query has more than NC); an edge whose candidates are all in the
                         // set already adds nothing
@@ -561,7 +564,12 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                         }
                         want = (em & ~L.cdone[qi]) != 0u;
                         if (want && !(vr & VR_COLLECTS)) {
-                            const EdgeCells ec = edge_cells(c.grid, c.cell_level, root_bb, entity_box(false, gm));
+                            bool in = (vr & VR_INSIDE) != 0u;
+                            if (!in) {
+                                const float4 rb = ldg4((const float4*)c.nodes);   // (root_bb's registers end above)
+                                in = box_has_point(rb, gm.x, gm.y) && box_has_point(rb, gm.z, gm.w);
+                            }
+                            const EdgeCells ec = edge_cells_inside(c.grid, c.cell_level, root_bb, gm, in);
                             if (ec.l > L.vdepth[qi]) {
                                 start[0] = collect_start(c, ec.l, ec.x0, ec.y0);
                                 if (ec.x0 != ec.x1 || ec.y0 != ec.y1) {

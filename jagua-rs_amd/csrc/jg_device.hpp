@@ -228,11 +228,11 @@ __device__ __forceinline__ int virtual_root_cells(const CdeView& c, float4 root,
     }
 }
 
-// The nodes from which the descent of an edge with bounding box eb, starting at a node n0 of depth
-// d0 that holds it, may start instead: the deepest nodes on the paths to its cells (edge_cells),
-// one or two of them (n1 = n0 then), when the cells lie below n0.
-__device__ __forceinline__ void edge_starts(const CdeView& c, float4 root, uint32_t d0, float4 eb, uint32_t& n0, uint32_t& n1) {
-    const EdgeCells e = edge_cells(c.grid, c.cell_level, root, eb);
+// The nodes from which the descent of an edge g (x1 y1 x2 y2), starting at a node n0 of depth d0 that
+// holds it, may start instead: the deepest nodes on the paths to its cells (edge_cells), one or
+// two of them (n1 = n0 then), when the cells lie below n0.  The edge lies inside the root box.
+__device__ __forceinline__ void edge_starts(const CdeView& c, float4 root, uint32_t d0, float4 g, uint32_t& n0, uint32_t& n1) {
+    const EdgeCells e = edge_cells_inside(c.grid, c.cell_level, root, g);
     if (e.l > d0) {
         n0 = cell_entry(c, e.l, e.x0, e.y0) & CELL_NODE;
         n1 = e.x0 != e.x1 || e.y0 != e.y1 ? cell_entry(c, e.l, e.x1, e.y1) & CELL_NODE : n0;

@@ -318,9 +318,9 @@ JG_HD HoldingCell holding_cell(const CellGrid& g, uint32_t level, float4 root, f
     return HoldingCell{level - s, x0 >> s, y0 >> s};
 }
 
-// The start cells of the descent of an edge with bounding box b, within the root box: the cell that
-// strictly holds it, or, deeper, the two cells of one level that share a side which the edge
-// crosses, (x0, y0) and (x1, y1) of level l (equal for one cell).
+// The start cells of the descent of an edge e (x1 y1 x2 y2): the cell that strictly holds it, or,
+// deeper, the two cells of one level that share a side which the edge crosses, (x0, y0) and
+// (x1, y1) of level l (equal for one cell).
 //
 // QTNode::collides reaches the deepest nodes on the paths to these cells and no others beside or
 // above them matter.  Every hazard present below a node is an entry of it (qt_node.rs:39-81:
@@ -336,17 +336,20 @@ JG_HD HoldingCell holding_cell(const CellGrid& g, uint32_t level, float4 root, f
 //  - below it, the edge leaves the node across that side only; its endpoint lies strictly inside the
 //    quadrant on the path, and the other three are disjoint, beyond the endpoint or the midline.
 // "Strictly" is by the margin of holding_cell, for the endpoints against the crossed side as well;
-// where it fails, one cell of a level above is taken.  An edge with a NaN lies inside no quadrant:
-// l = 0, no cell below the node that its descent starts from.
+// where it fails, one cell of a level above is taken.  All of it needs both endpoints inside the root
+// box: an edge that leaves it may reach no quadrant at all, and one with a NaN has an endpoint in none:
+// l = 0, no cell below the node that the descent starts from.
 struct EdgeCells {
     uint32_t l, x0, y0, x1, y1;
 };
-JG_HD EdgeCells edge_cells(const CellGrid& g, uint32_t level, float4 root, float4 b) {
+// ok: the endpoints are known to be inside the root box, but for a NaN.
+JG_HD EdgeCells edge_cells_inside(const CellGrid& g, uint32_t level, float4 root, float4 e, bool ok = true) {
+    const float4 b = make_float4(mn(e.x, e.z), mn(e.y, e.w), mx(e.x, e.z), mx(e.y, e.w));
     const float top = (float)((1u << level) - 1u);
     const uint32_t x0 = grid_index(b.x - g.eps - root.x, g.sx, top), x1 = grid_index(b.z + g.eps - root.x, g.sx, top);
     const uint32_t y0 = grid_index(b.y - g.eps - root.y, g.sy, top), y1 = grid_index(b.w + g.eps - root.y, g.sy, top);
     const uint32_t d = (x0 ^ x1) | (y0 ^ y1);
-    const bool ok = g.sx > 0.0f && b.x <= b.z && b.y <= b.w;
+    ok = ok && g.sx > 0.0f && !__builtin_isunordered(e.x, e.z) && !__builtin_isunordered(e.y, e.w);
     uint32_t s = !ok ? level : d ? 32u - (uint32_t)__builtin_clz(d) : 0u;
     EdgeCells o{level - s, x0 >> s, y0 >> s, x0 >> s, y0 >> s};
     if (s != 0u && ok) {
@@ -360,6 +363,9 @@ JG_HD EdgeCells edge_cells(const CellGrid& g, uint32_t level, float4 root, float
         if (t < s && sure) o = EdgeCells{level - t, x0 >> t, y0 >> t, x1 >> t, y1 >> t};
     }
     return o;
+}
+JG_HD EdgeCells edge_cells(const CellGrid& g, uint32_t level, float4 root, float4 e) {
+    return edge_cells_inside(g, level, root, e, box_has_point(root, e.x, e.y) && box_has_point(root, e.z, e.w));
 }
 
 // circle.rs:109-113 via edge.rs:63-87,153-159  Circle–Edge

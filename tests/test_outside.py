@@ -19,12 +19,12 @@ def _ring(x0, y0, x1, y1):
     return np.array([[x0, y0], [x1, y0], [x1, y1], [x0, y1]], np.float32)
 
 
-def _engines(hazards, depth=7):
+def _engines(hazards, depth=7, threshold=16):
     """Product and oracle engines of static hazards [(kind, vertices)] over BOX, after its exterior."""
     haz = [(O.KIND_EXTERIOR, _ring(*BOX))] + hazards
     cde = J.CDEngine(BOX, [J.Hazard(J.HazardEntity(k, i), J.SPolygon.new(v), False) for i, (k, v) in enumerate(haz)],
-                     J.CDEConfig(depth, 16, J.SPSurrogateConfig()))
-    return cde, O.OracleCDE.from_hazards(BOX, depth, 16, [(k, i, 0, v) for i, (k, v) in enumerate(haz)])
+                     J.CDEConfig(depth, threshold, J.SPSurrogateConfig()))
+    return cde, O.OracleCDE.from_hazards(BOX, depth, threshold, [(k, i, 0, v) for i, (k, v) in enumerate(haz)])
 
 
 def _mats(xy, rot=None):
@@ -54,8 +54,9 @@ def test_cells_outside_the_root_box(tmp_path):
     for seed in (1, 2):
         out = subprocess.run([str(exe), str(seed), "20000"], capture_output=True, text=True)
         assert out.returncode == 0, out.stdout + out.stderr
-        ok, outside, inside = out.stdout.split()[:3]
+        ok, outside, inside, leave, cells, nans = out.stdout.split()
         assert ok == "ok" and int(outside) > 100000 and int(inside) > 50000
+        assert int(leave) > 100000 and int(cells) > 20000 and int(nans) > 100000
 
 
 @pytest.mark.gpu
@@ -66,3 +67,27 @@ def test_collection_from_the_root_outside(cuda):
     cde, oc = _engines([(O.KIND_HOLE, arm)])
     ref = _check_sets(cuda, cde, oc, _ring(-2, -2, 2, 2), _mats([[-35, 8], [-35, 30], [-20, 50], [-60, 8], [5, 50], [-1, 20]]))
     assert ref["count"].tolist()[:3] == [2, 2, 2]
+
+
+@pytest.mark.gpu
+def test_collection_of_edges_outside(cuda):
+    """Queries in the notch of a hazard that reaches over the border, whose cells beside them are
+    Entire: their edges, outside the box, reach no node (the root itself does not collect)."""
+    notch = np.array([[-50, 20], [30, 20], [30, 80], [-50, 80], [-50, 60], [-2, 60], [-2, 40], [-50, 40]], np.float32)
+    cde, oc = _engines([(O.KIND_HOLE, notch)], threshold=2)
+    ref = _check_sets(cuda, cde, oc, _ring(-0.2, -0.2, 0.2, 0.2), _mats([[-8, 51.17], [-30, 48.83], [-2.5, 51.17], [-20, 30], [-1, 51.17]]))
+    assert ref["count"].tolist()[:3] == [1, 1, 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("depth,nv,r", [(7, 5, 2.0), (7, 24, 12.0), (10, 9, 5.0), (3, 40, 40.0)])
+def test_queries_around_the_border(cuda, depth, nv, r):
+    """Hazards across every border and in the middle, queries in and around the box."""
+    rng = np.random.default_rng(5 + depth)
+    c = np.concatenate([np.stack([rng.uniform(0, 100, 6), rng.choice([0.0, 100.0], 6)], 1),
+                        np.stack([rng.choice([0.0, 100.0], 6), rng.uniform(0, 100, 6)], 1), rng.uniform(0, 100, (6, 2))])
+    cde, oc = _engines([(O.KIND_HOLE, S.polygon(60 + i, 5, 20, 3.0, 20.0, i % 3) + p.astype(np.float32)) for i, p in enumerate(c)], depth)
+    n = 3000
+    mats = _mats(rng.uniform(-60, 160, (n, 2)), rng.uniform(0, 6.28, n))
+    ref = _check_sets(cuda, cde, oc, S.polygon(80 + nv, nv, nv, 0.5 * r, r, 2), mats)
+    assert len(np.unique(ref["count"])) > 2
