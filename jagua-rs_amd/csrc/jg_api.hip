@@ -141,6 +141,7 @@ static void set_view(jg_cde* c) {
     v.n_slots = (uint32_t)im.slot_ver.size();
     v.exterior_slot = c->exterior.idx;
     v.cd_threshold = c->cfg.cd_threshold;
+    v.box_bound = c->n_exterior == (c->map.valid(c->exterior) ? 1u : 0u) ? 1u : 0u;
     v.n_nodes = (uint32_t)im.nodes.size();
     v.ext_inner = make_float4(1.0f, 1.0f, 0.0f, 0.0f);
     if (c->map.valid(c->exterior)) {
@@ -762,6 +763,7 @@ static jg_hazkey cde_register(jg_cde* c, const jg_hazard_entity& ent, const Poly
     r.entity = ent;
     r.shape = shape;
     r.dynamic = dynamic;
+    if (!r.interior()) c->n_exterior++;
     const jg_hazkey k = c->map.insert(std::move(r));
     c->qt.register_hazard(0, root_entry(c->map.slots[k.idx].rec.shape, k), c->map);
     c->dirty = true;
@@ -804,7 +806,7 @@ extern "C" jg_status jg_cde_register_hazard(jg_cde* c, const jg_hazard_entity* e
 extern "C" jg_status jg_cde_deregister_hazard_by_key(jg_cde* c, jg_hazkey k) {
     if (!c) return fail(JG_ERR_INVALID_ARG, "null argument");
     if (!c->map.valid(k)) return fail(JG_ERR_NOT_REGISTERED, "Cannot deregister hazard that is not registered");
-    c->map.remove(k);
+    if (!c->map.remove(k).interior()) c->n_exterior--;
     c->qt.deregister_hazard(0, k.idx, k.version);
     c->dirty = true;
     return JG_OK;

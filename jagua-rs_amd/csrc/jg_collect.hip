@@ -20,7 +20,8 @@
 // coordinates' magnitude, far above the few ulps by which an Entire node or a quadrant flag may
 // stray past a box in f32.  The exterior hazard's Entire nodes lie outside the container, so it
 // can be ruled out only for an entity inside a box that is inside the container (the
-// container's bbox when it is an axis-aligned rectangle), shrunk by the same margin.
+// container's bbox when it is an axis-aligned rectangle), shrunk by the same margin.  An engine
+// with more hazards of exterior scope than that one skips nothing.
 //  - query edges: everything they can collect is an entry of the query's virtual root whose
 //    widened box meets the query's bbox.  Those candidates (up to NC) are listed per query when
 //    the pass starts, with each edge's mask of candidates its box meets; a visit is skipped
@@ -149,12 +150,6 @@ __device__ __forceinline__ bool boxes_meet(float4 a, float4 b) {
 __device__ __forceinline__ bool box_inside(float4 in, float4 out) {
     return in.x > out.x && in.z < out.z && in.y > out.y && in.w < out.w;
 }
-// Whether an entity with box eb may collect hazard `slot` anywhere below a node that holds it.
-__device__ __forceinline__ bool may_collect(const CdeView& c, uint32_t slot, float4 eb) {
-    if (slot == c.exterior_slot) return !box_inside(eb, inner_shrunk(c));
-    return boxes_meet(eb, widened(ldg4(c.haz_bbox + slot)));
-}
-
 // The node from which the descent towards cell (ix, iy) of level l may start, of an entity that visits
 // the nodes on the path to it one after another (edge_cells and circle_cells in jg_geom.hpp): the
 // first node on the path that collects, where the descent ends (QTNode::collect_collisions,
@@ -275,7 +270,7 @@ __device__ __forceinline__ void wave_collect(const CdeView& c, CollectLds& L, ui
             live = cnt > 0u;
             // a circle's start node is visited only if the circle meets its box (circle_cells)
             if (live && circle && (item & WL_NODE_MASK) != 0u) live = circle_box(g.x, g.y, g.z, nd.bbox);
-            if (live && em == SURR_MASK && cnt <= PRUNE_MAX) live = surrogate_live(c, L, nd, cnt, qs, entity_box(circle, g));
+            if (live && em == SURR_MASK && cnt <= PRUNE_MAX && c.box_bound) live = surrogate_live(c, L, nd, cnt, qs, entity_box(circle, g));
             if (live) {
                 if (nd.first_child >= 0 && nd.n_active_edges > c.cd_threshold) {
                     fc = nd.first_child;
@@ -418,7 +413,7 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
     for (uint32_t i = sub; i < SET_CAP; i += CG) L.set[qs * SET_CAP + i] = 0u;
     if (sub == 0) {
         L.ovf[qs] = 0u;
-        L.ncand[qs] = 0u;
+        L.ncand[qs] = c.box_bound ? 0u : NC + 1u;
         L.cdone[qs] = 0u;
     }
     int vr = 0;

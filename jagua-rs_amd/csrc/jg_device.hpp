@@ -93,6 +93,7 @@ struct CdeView {
     uint32_t n_slots, exterior_slot, cd_threshold, n_nodes;
     uint32_t cell_level;
     CellGrid grid;                    // the deepest table level's grid (circle_cells)
+    uint32_t box_bound;               // every hazard but exterior_slot's is collected only where its box is met
     float4 ext_inner;                 // a box inside the container (the exterior hazard's shape):
                                       // its bbox when that shape is an axis-aligned rectangle,
                                       // else empty (x_min > x_max)

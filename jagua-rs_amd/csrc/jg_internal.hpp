@@ -38,6 +38,7 @@ struct jg_cde {
     jg::SlotMap map;
     jg::QuadTree qt;
     jg_hazkey exterior{0, 0};
+    uint32_t n_exterior = 0;           // registered hazards of exterior scope
     bool dirty = true;
     bool dev_valid = false;
     jg::DevBlob dev;                   // the device image (pool order, with headroom)
