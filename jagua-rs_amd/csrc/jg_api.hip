@@ -548,8 +548,9 @@ __device__ __forceinline__ void collect_query(const CdeView& c, const ItemView& 
 }  // namespace
 
 // Hazard-collection queries of one item, one at a time per wavefront (persistent one-wavefront
-// workgroups).  Only for the engines and batches past the wave traversal's packed formats
-// (detect_direct_fits); k_collect_direct measured 1.4 to 2.7 times faster (collect_direct_launch).
+// workgroups).  For items that meet many hazards (expected_candidates), and the engines and batches past
+// the wave traversal's packed formats (detect_direct_fits); elsewhere k_collect_direct measured 1.4
+// to 2.7 times faster (collect_direct_launch).
 __global__ __launch_bounds__(64) void k_collect(CdeView c, ItemView it, const float* __restrict__ m6, uint64_t n,
                                                 uint32_t words, uint32_t cap, uint32_t* __restrict__ count,
                                                 uint64_t* __restrict__ hash, uint32_t* __restrict__ keys) {
@@ -565,17 +566,19 @@ __global__ __launch_bounds__(64) void k_collect(CdeView c, ItemView it, const fl
 }
 
 // The queries that k_collect_direct left with a count of COUNT_OVERFLOW, each collected by one wave with
-// the collector over every slot; a wave looks through 64 counts at a time.
+// the collector over every slot; the `share` waves of 64 queries take every share-th of them each.  (One
+// wave for 64 queries took up to 62 times one query's time, 40.6 ms instead of 0.85.)
 __global__ __launch_bounds__(64) void k_collect_rest(CdeView c, ItemView it, const float* __restrict__ m6, uint64_t n,
-                                                     uint32_t words, uint32_t cap, uint32_t* __restrict__ count,
+                                                     uint32_t share, uint32_t words, uint32_t cap, uint32_t* __restrict__ count,
                                                      uint64_t* __restrict__ hash, uint32_t* __restrict__ keys) {
     extern __shared__ uint32_t lds[];
     __shared__ uint32_t list[SET_LIST_CAP];
     __shared__ uint32_t list_n;
     const uint32_t lane = threadIdx.x;
     bool ready = false;
-    for (uint64_t q0 = (uint64_t)blockIdx.x * 64u; q0 < n; q0 += (uint64_t)gridDim.x * 64u) {
-        uint64_t left = __ballot(q0 + lane < n && count[q0 + lane] == COUNT_OVERFLOW);
+    const uint32_t turn = blockIdx.x % share;
+    for (uint64_t q0 = (uint64_t)(blockIdx.x / share) * 64u; q0 < n; q0 += (uint64_t)(gridDim.x / share) * 64u) {
+        uint64_t left = __ballot(lane % share == turn && q0 + lane < n && count[q0 + lane] == COUNT_OVERFLOW);
         if (left != 0ull && !ready) {
             for (uint32_t w = lane; w < words; w += 64) lds[w] = 0u;
             if (lane == 0) list_n = 0u;
@@ -758,12 +761,38 @@ extern "C" jg_status jg_spolygon_centroid(const jg_spolygon* p, float out[2]) {
 }
 
 // ------------------------------------------------------------------------------ ABI: engine
+static void count_hazard(jg_cde* c, const HazardRec& r, bool in) {
+    const float4 b = r.shape.bbox;
+    const double w = (double)b.z - b.x, h = (double)b.w - b.y, s = in ? 1.0 : -1.0;
+    if (!r.interior()) {
+        c->n_exterior += in ? 1u : ~0u;
+        return;
+    }
+    c->n_interior += in ? 1u : ~0u;
+    c->int_sides += s * (w + h);
+    c->int_area += s * w * h;
+}
+
+// How many candidates (hazards whose boxes its box meets) a query of `item` can be expected to have, its
+// placements and the hazards being spread over the container.  Where that nears what the wave
+// traversal's collector holds (16), most queries are left to the second launch, after the first one's
+// set-up, and the per-query kernel alone is faster.  us of 64 / 1000 / 10000 queries by k_collect, by
+// both launches: 5.5 expected 83 / 126 / 299, 56 / 95 / 144; 8.2 151 / 185 / 466, 58 / 207 / 321; 10
+// 130 / 151 / 386, 101 / 119 / 420; 16 158 / 221 / 509, 276 / 333 / 800; 23 225 / 246 / 653, 340 / 373 /
+// 952 (items of radius 60 to 250 over sheets of 300 and 2000).
+constexpr double COLLECT_DIRECT_MAX = 12.0;
+static double expected_candidates(const jg_cde* c, const jg_spolygon* item) {
+    const float4 b = item->poly.bbox, o = c->map.valid(c->exterior) ? c->map.slots[c->exterior.idx].rec.shape.bbox : c->qt.pool[0].bbox;
+    const double s = 0.5 * ((double)b.z - b.x + b.w - b.y), area = ((double)o.z - o.x) * ((double)o.w - o.y);
+    return (c->n_interior * s * s + s * c->int_sides + c->int_area) / area;
+}
+
 static jg_hazkey cde_register(jg_cde* c, const jg_hazard_entity& ent, const Polygon& shape, bool dynamic) {
     HazardRec r;
     r.entity = ent;
     r.shape = shape;
     r.dynamic = dynamic;
-    if (!r.interior()) c->n_exterior++;
+    count_hazard(c, r, true);
     const jg_hazkey k = c->map.insert(std::move(r));
     c->qt.register_hazard(0, root_entry(c->map.slots[k.idx].rec.shape, k), c->map);
     c->dirty = true;
@@ -806,7 +835,7 @@ extern "C" jg_status jg_cde_register_hazard(jg_cde* c, const jg_hazard_entity* e
 extern "C" jg_status jg_cde_deregister_hazard_by_key(jg_cde* c, jg_hazkey k) {
     if (!c) return fail(JG_ERR_INVALID_ARG, "null argument");
     if (!c->map.valid(k)) return fail(JG_ERR_NOT_REGISTERED, "Cannot deregister hazard that is not registered");
-    if (!c->map.remove(k).interior()) c->n_exterior--;
+    count_hazard(c, c->map.remove(k), false);
     c->qt.deregister_hazard(0, k.idx, k.version);
     c->dirty = true;
     return JG_OK;
@@ -978,13 +1007,15 @@ extern "C" jg_status jg_collect_batch(jg_cde* c, const jg_spolygon* item, const 
     int dev = 0, cus = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (detect_direct_fits(c, n)) {
+    if (detect_direct_fits(c, n) && !(expected_candidates(c, item) > COLLECT_DIRECT_MAX)) {
         s = collect_direct_launch(c->view, item->view, d_m6, n, d_keys ? capacity : 0u, d_count, d_hash, d_keys, (uint32_t)cus,
                                   (hipStream_t)stream);
         if (s != JG_OK) return s;
-        const uint64_t rest = std::min<uint64_t>((n + 63) / 64, (uint64_t)cus * 4u);
+        const uint64_t groups = (n + 63) / 64, waves = (uint64_t)cus * 16u;
+        const uint32_t share = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(waves / groups, 1u), 64u);
+        const uint64_t rest = std::min<uint64_t>(groups, waves) * share;
         hipLaunchKernelGGL(k_collect_rest, dim3((uint32_t)rest), dim3(64), (size_t)words * 4, (hipStream_t)stream, c->view,
-                           item->view, d_m6, n, words, d_keys ? capacity : 0u, d_count, d_hash, d_keys);
+                           item->view, d_m6, n, share, words, d_keys ? capacity : 0u, d_count, d_hash, d_keys);
         HIP_TRY(hipGetLastError());
         return JG_OK;
     }

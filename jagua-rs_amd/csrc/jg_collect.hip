@@ -482,6 +482,11 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
         }
     }
     wave_sync();
+    // without a list, a query that may outgrow its set is left before any work is spent on it
+    if (DIRECT) {
+        if (active && sub == 0 && L.ncand[qs] > SET_CAP) L.ovf[qs] = 1u;
+        wave_sync();
+    }
     if (active) {
         // a pre-seeded collector, then the exterior when the shape leaves the engine's bbox
         // (cd_engine.rs:262-264); the traversal goes on regardless
@@ -621,7 +626,7 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
         const float2 qpoi = xform(m, it.poi.x, it.poi.y);
         const uint32_t nc = L.ncand[qs];
         const bool listed = nc <= NC;
-        const uint32_t n_scan = listed ? nc : vcnt;
+        const uint32_t n_scan = listed ? nc : DIRECT ? 0u : vcnt;
         for (uint32_t k0 = 0; k0 < n_scan; k0 += CG) {
             const uint32_t k = k0 + sub;
             uint32_t sl = 0;
@@ -643,6 +648,37 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
                 }
             }
             containment_group(c, L, it, m, bb, qpoi, qs, sub, lane, pend, sl, rel);
+        }
+    }
+    // few queries in a pass: with more than NC candidates the virtual root's entries are scanned by the
+    // whole wave, as a shallow one has up to every hazard of the layout.  us by the query's CG lanes /
+    // by the wave, items of radius 60 over the 2000-item sheet: 64 queries 82 / 56, 1000 284 / 95,
+    // 10000 333 / 144.  (Not in the plan's passes of CP queries, where it spills 11 more registers.)
+    for (uint32_t q = 0; DIRECT && q < P; q++) {
+        if (L.ncand[q] <= NC || L.ovf[q]) continue;
+        const Mat mq{L.mat[q][0], L.mat[q][1], L.mat[q][2], L.mat[q][3], L.mat[q][4], L.mat[q][5]};
+        const float4 bq = L.qbox[q];
+        const float2 pq = xform(mq, it.poi.x, it.poi.y);
+        const uint32_t n_scan = L.vcnt[q], e0 = L.vbeg[q];
+        for (uint32_t k0 = 0; k0 < n_scan; k0 += WAVE) {
+            const uint32_t k = k0 + lane;
+            const uint32_t sf = k < n_scan ? ldg_slot_flags(c.ent + e0 + k) : ENTIRE_BIT;
+            const uint32_t sl = sf & SLOT_MASK;
+            int rel = REL_DISJOINT;
+            bool pend = false;
+            if (!(sf & ENTIRE_BIT) && !set_has(L, q, sl)) {
+                rel = box_almost_relation(ldg4(c.haz_bbox + sl), bq);
+                if (rel == REL_SURROUNDING || rel == REL_ENCLOSED) pend = true;
+                else if (ldg4(c.haz_poi + sl).w == 0.0f) set_put(L, q, sl);
+            }
+            for (uint64_t pm = __ballot(pend); pm; pm &= pm - 1ull) {
+                const int l = __builtin_ctzll(pm);
+                const uint32_t s2 = (uint32_t)__shfl((int)sl, l, 64);
+                const float4 hp = ldg4(c.haz_poi + s2);
+                const bool contained = __shfl(rel, l, 64) == REL_SURROUNDING ? pip_hazard_wave(c, s2, pq.x, pq.y, lane)
+                                                                             : pip_query_wave(it, mq, bq, hp.x, hp.y, lane);
+                if (lane == (uint32_t)l && (hp.w != 0.0f ? contained : !contained)) set_put(L, q, s2);
+            }
         }
     }
     wave_sync();

@@ -39,6 +39,8 @@ struct jg_cde {
     jg::QuadTree qt;
     jg_hazkey exterior{0, 0};
     uint32_t n_exterior = 0;           // registered hazards of exterior scope
+    uint32_t n_interior = 0;           // those of interior scope, and over them the sums of
+    double int_sides = 0.0, int_area = 0.0;   // their boxes' sides (width plus height) and areas
     bool dirty = true;
     bool dev_valid = false;
     jg::DevBlob dev;                   // the device image (pool order, with headroom)

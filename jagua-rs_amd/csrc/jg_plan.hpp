@@ -180,7 +180,7 @@ jg_status collect_launch(const TableLayout& L, uint8_t* base, const float* d_m6,
                          uint64_t* d_hash, uint32_t* d_keys, uint64_t* ovf, uint32_t n_cus, hipStream_t stream);
 
 // The batched collection over one set, described by value: no table, no allocation.  A query whose
-// set outgrows the batched kernel's collector is left with a count of COUNT_OVERFLOW.
+// set may outgrow the batched kernel's collector is left with a count of COUNT_OVERFLOW.
 constexpr uint32_t COUNT_OVERFLOW = 0xffffffffu;
 jg_status collect_direct_launch(const CdeView& cde, const ItemView& item, const float* d_m6, uint64_t n, uint32_t cap,
                                 uint32_t* d_count, uint64_t* d_hash, uint32_t* d_keys, uint32_t n_cus, hipStream_t stream);
