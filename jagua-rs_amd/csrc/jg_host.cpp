@@ -746,6 +746,13 @@ void fill_cells(PoolImage& im, const QuadTree& qt, int32_t n, uint32_t depth, ui
     fill_cells(im, qt, ch + 2, depth + 1, level + 1, 2 * ix, 2 * iy, cdepth);
     fill_cells(im, qt, ch + 3, depth + 1, level + 1, 2 * ix + 1, 2 * iy, cdepth);
 }
+// Adds the nodes under n (at depth `depth`) of each depth within the tables' levels to count.
+void count_depths(const QuadTree& qt, int32_t n, uint32_t depth, uint64_t* count) {
+    count[depth]++;
+    const int32_t ch = qt.pool[(size_t)n].child;
+    if (ch < 0 || depth == CELL_LEVELS_MAX) return;
+    for (int k = 0; k < 4; k++) count_depths(qt, ch + k, depth + 1, count);
+}
 }  // namespace
 
 void image_cells(PoolImage& im, const QuadTree& qt) {
@@ -753,6 +760,12 @@ void image_cells(PoolImage& im, const QuadTree& qt) {
     // a degenerate root box has no usable grid: level 0 only, the root
     const bool flat = !(r.z > r.x && r.w > r.y);
     im.cell_level = flat ? 0u : std::min<uint32_t>(qt.pool[0].level, CELL_LEVELS_MAX);
+    if (im.cell_level > CELL_LEVELS_MIN) {
+        uint64_t count[CELL_LEVELS_MAX + 1] = {};
+        count_depths(qt, 0, 0, count);
+        while (im.cell_level > CELL_LEVELS_MIN && count[im.cell_level] * CELL_LEVEL_SHARE < (uint64_t)1 << (2 * im.cell_level))
+            im.cell_level--;
+    }
     im.cells.assign((((size_t)1 << (2 * (im.cell_level + 1))) - 1) / 3, 0u);
     fill_cells(im, qt, 0, 0, 0, 0, 0, CELL_NO_CDEPTH);
 }

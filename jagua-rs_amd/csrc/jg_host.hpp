@@ -87,11 +87,16 @@ struct QEntry {                          // QTHazard in one node (qt_hazard.rs:1
     std::vector<uint32_t> edges;         // edge indices into the hazard polygon
 };
 
-// Deepest level of the cell tables: the tree's depth, at most this (levels 0 .. 9: 1.4 MB).  A pole starts at
-// its cell's node, so each level saves a visit per pole: us per step at 7 / 8 / 9 levels 679 / 643 /
-// 645 (2000-item sheet, depth 8) and 436 / 413 / 398 (2500 concave items, depth 10); the update of
-// one placed item takes 96 us instead of 95.
-constexpr uint32_t CELL_LEVELS_MAX = 9;
+// Deepest level of the cell tables: the tree's depth, at most CELL_LEVELS_MAX (levels 0 .. 9: 1.4 MB), and
+// beyond CELL_LEVELS_MIN (87 KB) only where at least one cell in CELL_LEVEL_SHARE has a node of its
+// level.  A pole starts at its cell's node, so in a full layout each level saves a visit per pole: us
+// per step at 7 / 8 / 9 levels 679 / 643 / 645 (2000-item sheet, depth 8) and 436 / 413 / 398 (2500
+// concave items, depth 10), where the update of one placed item takes 96 us instead of 95.  In a
+// sparse one an update rewrites the cells under large empty nodes: one item put into and taken
+// out of an otherwise empty container, depth 10, took 222 us with 9 levels and 125 with 7, its
+// first upload 1326 and 652.  The share is 0.2 to 0.4 in full layouts and below 0.05 with a
+// container and a few holes alone.  A full build decides; patches keep its levels.
+constexpr uint32_t CELL_LEVELS_MAX = 9, CELL_LEVELS_MIN = 7, CELL_LEVEL_SHARE = 16;
 constexpr uint32_t CELL_NO_CDEPTH = 15;
 
 struct QNode {                           // QTNode (qt_node.rs:14-25)

@@ -244,3 +244,18 @@ def test_start_cells(tmp_path):
         assert out.returncode == 0, out.stdout + out.stderr
         ok, leaves, on, two = out.stdout.split()
         assert ok == "ok" and int(leaves) > 10000 and int(on) > 30000 and int(two) > 5000
+
+
+def test_cell_table_levels(tmp_path):
+    """Full layouts get the deep cell tables, sparse ones the shallow ones, and patches leave
+    every entry right at any number of levels (tests/cell_levels_check.cpp)."""
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = tmp_path / "cell_levels_check"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", os.path.join(root, "tests", "cell_levels_check.cpp"),
+                    os.path.join(root, "jagua-rs_amd", "csrc", "jg_host.cpp"), "-o", str(exe)],
+                   check=True, capture_output=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.startswith("ok"), out.stdout + out.stderr
