@@ -46,15 +46,18 @@ DevBlob::~DevBlob() {
 }
 jg_status DevBlob::reserve(size_t bytes) {
     if (bytes <= cap) return JG_OK;
+    return reserve_exact(bytes < 4096 ? 4096 : bytes + bytes / 4);
+}
+jg_status DevBlob::reserve_exact(size_t bytes) {
+    if (bytes <= cap) return JG_OK;
     if (ptr) {
         HIP_TRY(hipDeviceSynchronize());
         HIP_TRY(hipFree(ptr));
         ptr = nullptr;
         cap = 0;
     }
-    size_t c = bytes < 4096 ? 4096 : bytes + bytes / 4;
-    HIP_TRY(hipMalloc(&ptr, c));
-    cap = c;
+    HIP_TRY(hipMalloc(&ptr, bytes));
+    cap = bytes;
     return JG_OK;
 }
 

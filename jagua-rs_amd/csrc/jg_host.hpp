@@ -201,6 +201,16 @@ void image_cells(PoolImage& im, const QuadTree& qt);
 // Whether QTNode::collect_collisions tests node n's entries (qt_node.rs:151-191).
 bool collects_at(const QuadTree& qt, int32_t n);
 
+// Workgroups of a launch that claims its jobs from a counter, so that any number of them finishes it:
+// `want`, halved until alloc(fixed + per * workgroups) gives the memory they work in; 0 when it
+// gives it for none.
+template <class Alloc>
+uint32_t fit_workgroups(uint32_t want, uint64_t fixed, uint64_t per, Alloc alloc) {
+    for (uint32_t g = want; g > 0; g /= 2)
+        if (alloc(fixed + per * (uint64_t)g)) return g;
+    return 0;
+}
+
 // Full build of the host mirror and the device layout (capacities with headroom).
 void image_build(PoolImage& im, QuadTree& qt, const SlotMap& map);
 // Rewrites the nodes and slots changed since the last build or patch into the host mirror and

@@ -16,7 +16,8 @@ struct DevBlob {                       // one device allocation, grown on demand
     DevBlob(const DevBlob&) = delete;
     DevBlob& operator=(const DevBlob&) = delete;
     ~DevBlob();
-    jg_status reserve(size_t bytes);
+    jg_status reserve(size_t bytes);       // with room to grow
+    jg_status reserve_exact(size_t bytes);
 };
 
 jg_status fail(jg_status code, const std::string& msg);

@@ -479,7 +479,7 @@ extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offs
     // 24 / 35 / 61, 192 of 8-256 vertices 4.1 / 4.4 / 5.9, 1500 of them 12.0 / 10.1 / 12.5, 4000
     // concave ones of 64-1024 vertices 66 / 61 / 59.
     const bool wide = n_polys <= 2u * (uint32_t)cus;
-    const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(n_polys, (wide ? 2u : 3u) * (uint32_t)cus));
+    const uint32_t want = std::max<uint32_t>(1u, std::min<uint32_t>(n_polys, (wide ? 2u : 3u) * (uint32_t)cus));
 
     const size_t b_jobs = sizeof(PoleJob) * n_polys;
     const size_t o_verts = (b_jobs + 255) & ~(size_t)255;
@@ -488,10 +488,15 @@ extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offs
     const size_t o_st = (o_np + 4 * (size_t)n_polys + 255) & ~(size_t)255;
     const size_t o_ctr = (o_st + 4 * (size_t)n_polys + 255) & ~(size_t)255;
     const size_t o_fr = o_ctr + 256;
-    const size_t total = o_fr + sizeof(PoleSpill) * (size_t)grid;
+    // 1.15 MB per workgroup for the length of the call, 0.88 GB at most; fewer workgroups where the
+    // device has less to give
     DevBlob blob;
-    st = blob.reserve(total);
-    if (st != JG_OK) return st;
+    const uint32_t grid = fit_workgroups(want, o_fr, sizeof(PoleSpill), [&](uint64_t bytes) {
+        st = blob.reserve_exact((size_t)bytes);
+        if (st != JG_OK) (void)hipGetLastError();     // or the launch below would report it
+        return st == JG_OK;
+    });
+    if (grid == 0) return st;
     uint8_t* base = (uint8_t*)blob.ptr;
     st = hip_check(hipMemcpy(base, jobs.data(), b_jobs, hipMemcpyHostToDevice), "hipMemcpy pole jobs");
     if (st == JG_OK)
