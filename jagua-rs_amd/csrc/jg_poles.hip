@@ -80,8 +80,9 @@ struct PoleArgs {
     uint32_t* n_poles;
     uint32_t* status;
     PoleSpill* spill;         // [grid]
-    uint32_t* counter;
+    uint32_t* counter;        // jobs taken, trees emptied
     uint32_t n_jobs, pole_cap, surrogate;
+    uint32_t blocks;          // node blocks per tree, at most NODE_CAP / 4
     uint32_t lim_n[3];
     float lim_cov[3];
 };
@@ -136,6 +137,7 @@ struct PoleSearch {
     const PoleJob job;
     const float2* gv;          // its vertices
     const float4* gP;          // its poles
+    const uint32_t blocks;     // of its tree
     const uint32_t tid, lane, wv;
 
     __device__ float4 box(uint32_t b, uint32_t i) const { return i < FL ? L.box[b][i] : S.box[b][i]; }
@@ -294,12 +296,12 @@ struct PoleSearch {
                     uint32_t blk = link & PN_CHILD;
                     if (blk == 0u) {
                         blk = atomicAdd(&L.n_blocks, 1u);
-                        if (blk < NODE_CAP / 4u) {
+                        if (blk < blocks) {
                             S.nodes[ni].link = link | blk;
                             for (uint32_t k = 0; k < 4u; k++) S.nodes[4u * blk + k] = PoleNode{0.0f, PN_NEW};
                         }
                     }
-                    if (blk < NODE_CAP / 4u) {
+                    if (blk < blocks) {
                         const float4 b = box(cur, i);
                         const uint32_t o = 4u * (at + lanes_below(sp, lane));
                         for (uint32_t k = 0; k < 4u; k++) put_cell(cur ^ 1u, o + k, box_quadrant(b, (int)k), 4u * blk + k);
@@ -308,7 +310,7 @@ struct PoleSearch {
                 at += (uint32_t)__builtin_popcountll(sp);
             }
             __syncthreads();
-            if (L.n_blocks > NODE_CAP / 4u) return PJ_FULL;
+            if (L.n_blocks > blocks) return PJ_FULL;
             cur ^= 1u;
             nF = tot * 4u;
         }
@@ -376,21 +378,26 @@ __global__ __launch_bounds__(NT) void k_poles(PoleArgs a) {
         if (j >= a.n_jobs) return;
         const PoleJob job = a.jobs[j];
         float4* P = a.poles + (size_t)job.out * a.pole_cap;
-        PoleSearch<NT, FL, VL> ps{L, a.spill[blockIdx.x], job, a.verts + job.v_begin, P, tid, tid & 63u, tid >> 6};
+        PoleSearch<NT, FL, VL> ps{L, a.spill[blockIdx.x], job, a.verts + job.v_begin, P, a.blocks, tid, tid & 63u, tid >> 6};
         if (job.n <= VL)
             for (uint32_t k = tid; k < job.n; k += NT) L.v[k] = ps.gv[k];
         ps.start();
         float covered = 0.0f;
         uint32_t np = 0, st;
+        bool emptied = false;
         for (;;) {
             float4 best = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             __syncthreads();                              // the pole (or the new tree) of the last round
             st = ps.search(np, best);
-            if (st == PJ_FULL) {
+            if (st == PJ_FULL && !emptied) {              // an empty tree holds any search
                 __syncthreads();
                 ps.start();
+                if (tid == 0) atomicAdd(&a.counter[1], 1u);
+                emptied = true;
                 continue;
             }
+            emptied = false;
+            if (st == PJ_FULL) st = PJ_HOST;              // (but for the smaller trees of the tests)
             if (st != PJ_OK) break;
             if (tid == 0) {
                 P[np] = best;
@@ -435,9 +442,9 @@ void parallel_for(size_t n, F fn) {
 
 }  // namespace
 
-extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offsets, uint32_t n_polys,
-                                           const jg_surrogate_config* cfg, jg_spolygon** out,
-                                           uint32_t* n_host_completed) {
+// blocks: node blocks per cell tree; n_emptied (may be null): how many trees were full and emptied.
+static jg_status new_batch(const float* xy, const uint32_t* offsets, uint32_t n_polys, const jg_surrogate_config* cfg,
+                           jg_spolygon** out, uint32_t* n_host_completed, uint32_t blocks, uint32_t* n_emptied) {
     if (!out || (n_polys && (!xy || !offsets))) return fail(JG_ERR_INVALID_ARG, "null argument");
     if (n_host_completed) *n_host_completed = 0;
     if (n_polys == 0) return JG_OK;
@@ -512,6 +519,7 @@ extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offs
     a.status = (uint32_t*)(base + o_st);
     a.spill = (PoleSpill*)(base + o_fr);
     a.counter = (uint32_t*)(base + o_ctr);
+    a.blocks = blocks;
     a.n_jobs = n_polys;
     a.pole_cap = pole_cap;
     a.surrogate = cfg ? 1u : 0u;
@@ -531,6 +539,7 @@ extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offs
     if (st == JG_OK) st = hip_check(hipMemcpy(np.data(), base + o_np, 4 * (size_t)n_polys, hipMemcpyDeviceToHost), "hipMemcpy");
     if (st == JG_OK)
         st = hip_check(hipMemcpy(status.data(), base + o_st, 4 * (size_t)n_polys, hipMemcpyDeviceToHost), "hipMemcpy");
+    if (st == JG_OK && n_emptied) st = hip_check(hipMemcpy(n_emptied, base + o_ctr + 4, 4, hipMemcpyDeviceToHost), "hipMemcpy");
     if (st != JG_OK) return st;
 
     // finish: the POI, the surrogate from its poles; polygons whose search outgrew the device
@@ -588,4 +597,19 @@ extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offs
     }
     if (n_host_completed) *n_host_completed = n_host;
     return JG_OK;
+}
+
+extern "C" jg_status jg_spolygon_new_batch(const float* xy, const uint32_t* offsets, uint32_t n_polys,
+                                           const jg_surrogate_config* cfg, jg_spolygon** out,
+                                           uint32_t* n_host_completed) {
+    return new_batch(xy, offsets, n_polys, cfg, out, n_host_completed, NODE_CAP / 4u, nullptr);
+}
+
+// For the tests, which no polygon takes to a full tree: jg_spolygon_new_batch with trees of `blocks`
+// node blocks.  A search that a smaller tree cannot hold is left to the host routine.
+extern "C" jg_status jg_check_spolygon_new_batch(const float* xy, const uint32_t* offsets, uint32_t n_polys,
+                                                 const jg_surrogate_config* cfg, jg_spolygon** out,
+                                                 uint32_t* n_host_completed, uint32_t blocks, uint32_t* n_emptied) {
+    if (blocks < 1u || blocks > NODE_CAP / 4u || !n_emptied) return fail(JG_ERR_INVALID_ARG, "tree size out of range");
+    return new_batch(xy, offsets, n_polys, cfg, out, n_host_completed, blocks, n_emptied);
 }
