@@ -961,8 +961,9 @@ static jg_status check_item(const jg_spolygon* item, uint32_t flags) {
     return JG_OK;
 }
 
-extern "C" jg_status jg_detect_batch(jg_cde* c, const jg_spolygon* item, const float* d_m6, uint64_t n,
-                                     const jg_hazard_filter* filter, uint32_t flags, uint8_t* d_status, void* stream) {
+// plain: by k_detect_plain, whatever the engine and the batch.
+static jg_status detect_batch(jg_cde* c, const jg_spolygon* item, const float* d_m6, uint64_t n,
+                              const jg_hazard_filter* filter, uint32_t flags, uint8_t* d_status, void* stream, bool plain) {
     if (!c || !item) return fail(JG_ERR_INVALID_ARG, "null argument");
     if (n == 0) return JG_OK;
     if (!d_m6 || !d_status) return fail(JG_ERR_INVALID_ARG, "null device buffer");
@@ -981,7 +982,7 @@ extern "C" jg_status jg_detect_batch(jg_cde* c, const jg_spolygon* item, const f
     const uint32_t block = 256;
     const uint64_t grid = (n + block - 1) / block;
     if (grid > 0x7fffffffull) return fail(JG_ERR_INVALID_ARG, "batch too large");
-    if (detect_direct_fits(c, n)) {
+    if (!plain && detect_direct_fits(c, n)) {
         s = detect_direct_launch(c->view, iv, fv, flags, d_m6, n, d_status, (hipStream_t)stream);
         if (s != JG_OK) return s;
     } else {
@@ -991,6 +992,19 @@ extern "C" jg_status jg_detect_batch(jg_cde* c, const jg_spolygon* item, const f
     }
     if (fv.kind == 1) return filter_read_done(c, (hipStream_t)stream);
     return JG_OK;
+}
+
+extern "C" jg_status jg_detect_batch(jg_cde* c, const jg_spolygon* item, const float* d_m6, uint64_t n,
+                                     const jg_hazard_filter* filter, uint32_t flags, uint8_t* d_status, void* stream) {
+    return detect_batch(c, item, d_m6, n, filter, flags, d_status, stream, false);
+}
+
+// For the tests, whose engines and batches are all within the wave traversal's formats: jg_detect_batch
+// by the kernel that takes those past them.
+extern "C" jg_status jg_check_detect_batch_plain(jg_cde* c, const jg_spolygon* item, const float* d_m6, uint64_t n,
+                                                 const jg_hazard_filter* filter, uint32_t flags, uint8_t* d_status,
+                                                 void* stream) {
+    return detect_batch(c, item, d_m6, n, filter, flags, d_status, stream, true);
 }
 
 extern "C" jg_status jg_collect_batch(jg_cde* c, const jg_spolygon* item, const float* d_m6, uint64_t n,
