@@ -653,8 +653,11 @@ uint32_t table_chunk(const jg_plan_config& cfg, uint64_t n_all, uint32_t n_cus, 
 }
 
 // What the sets' compact table counts against JG_NOALLOC_SCRATCH_BYTES, whatever the schedule's
-// defaults choose: descriptors, units, COMPACT_FIXED bytes of counters and bases, groups.
-constexpr size_t COMPACT_FIXED = 3360;
+// defaults choose: descriptors, units, COMPACT_FIXED bytes of counters and bases, groups.  The limit is
+// part of the interface, so it counts what the first form of the table had, three counters for
+// each of 8 streams and two more, a line each, and 8 bases, not what a later form has.
+constexpr size_t COMPACT_FIXED = 4u * STREAM_STRIDE * (3u * 8u + 2u) + 4u * 8u;
+static_assert(COMPACT_FIXED == 3360u, "calls near the limit would change sides");
 uint64_t compact_table_bytes(const std::vector<jg_query_set>& sets, const jg_plan_config& cfg) {
     const uint32_t uq = table_chunk(cfg, 0, 0, true);
     uint64_t units = 0, groups = 0;

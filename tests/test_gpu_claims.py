@@ -62,3 +62,24 @@ def test_noalloc_takes_what_its_scratch_was_sized_for(cuda, layout, item):
     got = out.cpu().numpy()
     np.testing.assert_array_equal(got[:n], np.tile(ref, n // 40000 + 1)[:n])
     assert (got[n:] == 99).all()
+
+
+@pytest.mark.parametrize("item,n_sets,chunk,most", [(0, 1, 0, 7894076), (1, 1, 0, 4066590), (2, 1, 0, 4066302),
+                                                    (2, 3, 0, 4066204), (2, 1, 16, 3727422)])
+def test_noalloc_limit_to_the_query(cuda, layout, item, n_sets, chunk, most):
+    """The largest call that the fixed scratch takes is part of the interface: descriptors, the item's
+    record, a unit per 64 queries (or the chunk) and a group per 8 or 2, whatever form the table has."""
+    cde, oc, prod, orc, box = layout
+    cde.sync()
+    m = torch.zeros((most + 1, 6), dtype=torch.float32, device=cuda)
+    out = torch.empty(most + 1, dtype=torch.uint8, device=cuda)
+
+    def call(n):
+        per = n // n_sets
+        J.detect_sets_noalloc([(cde, prod[item], k * per, per if k < n_sets - 1 else n - per * k, None) for k in range(n_sets)],
+                              m, out, chunk=chunk)
+
+    call(most)
+    with pytest.raises(J.JaguaError, match="scratch"):
+        call(most + 1)
+    torch.cuda.synchronize()
