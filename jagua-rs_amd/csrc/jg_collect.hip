@@ -482,12 +482,9 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
         }
     }
     wave_sync();
-    // without a list, a query that may outgrow its set is left before any work is spent on it
-    if (DIRECT) {
-        if (active && sub == 0 && L.ncand[qs] > SET_CAP) L.ovf[qs] = 1u;
-        wave_sync();
-    }
     if (active) {
+        // without a list, a query that may outgrow its set is left before any work is spent on it
+        if (DIRECT && sub == 0 && L.ncand[qs] > SET_CAP) L.ovf[qs] = 1u;
         // a pre-seeded collector, then the exterior when the shape leaves the engine's bbox
         // (cd_engine.rs:262-264); the traversal goes on regardless
         for (uint32_t i = sub; i < sd.n_seed; i += CG) set_put(L, qs, ldg1(sd.seed + i));
