@@ -556,7 +556,10 @@ jg_status detect_direct_launch(const CdeView& cde, const ItemView& item, const F
     // keep the launch within that many, up to 16, as a wave's time grows with its queries long
     // before its lanes are full; 32 and 64, which fill them, once the launch is three times that deep
     // at 16 and at 32, but for filtered queries of large items, whose polygon stages then make the
-    // tail (300 vertices, 500000 queries: 549 us at 16, 600 at 32; without a filter 297 and 222).
+    // tail.  That line is on the safe side: us at 16 / at up to 64 of 500000 filtered queries, two
+    // star-shaped items 358 / 311 and 362 / 304 at 65 vertices, 476 / 450 and 444 / 403 at 160, 551 / 602
+    // and 591 / 607 at 300, 949 / 1052 and 900 / 1049 at 800; two concave ones 312 / 199 and 530 / 535 at 65,
+    // 373 / 273 and 982 / 1069 at 300 (without a filter a star-shaped one of 300 takes 297 and 222).
     // us at 1 / 2 / 4 / 16 / 32 / 64 queries per wave (2000-item layout, 64-vertex item):
     // 1000 queries 18 / 20 / 21 / 26 / 32 / 41, 5000 34 / 35 / 34 / 39 / 47 / 62, 16384 49 / 40 / 36 / 41 / 49 /
     // 61, 65536 154 / 100 / 76 / 73 / 77 / 101, 262144 548 / 338 / 217 / 130 / 114 / 108,
@@ -633,9 +636,12 @@ uint32_t table_lanes(const jg_plan_config& cfg, uint32_t v, uint64_t n_all, uint
     } else if (lanes == 0) {
         // by vertices in a large launch: us per step at up to 32 lanes (the vertices rounded up) / at
         // these / at 64 for all above 32, 552 / 539 / 592 (2000-item sheet), 363 / 333 / 345
-        // (concave items of 300 vertices at the mean).  A launch with waves to spare, a query
-        // or less for each after the surrogate stage: the whole wave, as its time is a pass's
-        // (32000 queries of 64 items of 8-512 vertices: 93 -> 81 us).
+        // (concave items of 300 vertices at the mean).  At the edges, us at 8 / 16 / 32 / 64 lanes (16
+        // items of one size, 524288 queries): 16 vertices 159 / 160 / 180 / 217, 17 169 / 162 / 174 / 207,
+        // 64 208 / 189 / 193 / 227, 65 214 / 193 / 199 / 239, 96 244 / 220 / 222 / 259, 200 356 / 301 / 277 / 309,
+        // 384 516 / 406 / 356 / 363, 512 633 / 482 / 405 / 403, 768 876 / 640 / 511 / 476.  A launch with
+        // waves to spare, a query or less for each after the surrogate stage: the whole wave, as its
+        // time is a pass's (32000 queries of 64 items of 8-512 vertices: 93 -> 81 us).
         lanes = v <= 16u ? 8u : v <= 64u ? 16u : v <= 384u ? 32u : 64u;
         if (n_all <= (uint64_t)n_cus * 160u) lanes = 64u;
     }

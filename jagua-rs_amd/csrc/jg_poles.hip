@@ -15,8 +15,8 @@
 // poles alone, and a cell's distance to the border does not depend on them.  So the cells are
 // kept as a tree over the polygon's searches (PoleNode): a cell met before costs the poles added
 // since, a new one its edges, split over the lanes that the level's new cells leave free.
-// 192 polygons of 8-256 vertices took 110 ms with every cell evaluated anew by one thread and take
-// 4.1 ms; one polygon of 1024 vertices 1800 and 24 ms.
+// A call with 192 polygons of 8-256 vertices took 108 ms with every cell evaluated anew by one thread and
+// takes 5.8 ms, 3.8 of it here; one with a polygon of 1024 vertices 1800 and 27 ms.
 //
 // The arithmetic per edge and pole is pole_cell's (jg_geom.hpp).  Minima may be taken in any
 // order, the square root of the least squared distance is the least distance (sqrtf is
@@ -482,9 +482,9 @@ static jg_status new_batch(const float* xy, const uint32_t* offsets, uint32_t n_
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     // 1024 threads per polygon while every polygon has half a compute unit to itself, as its chain
     // of levels is what takes the time; 512 where polygons queue, as the lanes that a short level
-    // leaves idle are then missed.  ms at 1024 / 512 / 256 threads: one polygon of 1024 vertices
-    // 24 / 35 / 61, 192 of 8-256 vertices 4.1 / 4.4 / 5.9, 1500 of them 12.0 / 10.1 / 12.5, 4000
-    // concave ones of 64-1024 vertices 66 / 61 / 59.
+    // leaves idle are then missed.  ms per call at 1024 / 512 threads: one polygon of 1024 vertices 26.9 /
+    // 37.7, 192 of 8-256 vertices 5.3 / 6.0, 513 of them 5.9 / 6.5, 1500 11.2 / 9.8, 2000 concave ones
+    // of 64-1024 vertices 37.2 / 35.7.  (256 threads, measured earlier: 61 for the first, 12.5 for the 1500.)
     const bool wide = n_polys <= 2u * (uint32_t)cus;
     const uint32_t want = std::max<uint32_t>(1u, std::min<uint32_t>(n_polys, (wide ? 2u : 3u) * (uint32_t)cus));
 
