@@ -360,22 +360,21 @@ __device__ __forceinline__ uint64_t group_sum_u64(uint64_t v) {
 }
 
 // detect_containment_collision (cd_engine.rs:231-255) for one candidate of the query, by the
-// query's CG lanes (the one holding it in `pend`): inserts it when it collides.
+// n_lanes lanes from gbase on (the one holding it in `pend`): inserts it when it collides.
 __device__ __forceinline__ void containment_group(const CdeView& c, CollectLds& L, const ItemView& it, const Mat& m,
-                                                  float4 bb, float2 qpoi, uint32_t qs, uint32_t sub, uint32_t lane,
-                                                  bool pend, uint32_t sl, int rel) {
-    const uint64_t gmask = (1ull << CG) - 1ull;
-    const uint32_t gbase = qs * CG;
+                                                  float4 bb, float2 qpoi, uint32_t qs, uint32_t sub, uint32_t n_lanes,
+                                                  uint32_t gbase, uint32_t lane, bool pend, uint32_t sl, int rel) {
+    const uint64_t gmask = ~0ull >> (WAVE - n_lanes);
     for (uint64_t pm = (ballot(pend) >> gbase) & gmask; pm; pm &= pm - 1ull) {
         const int l = (int)gbase + __builtin_ctzll(pm);
         const uint32_t s2 = (uint32_t)__shfl((int)sl, l, 64);
         const int rl = __shfl(rel, l, 64);
         bool contained;
         if (rl == REL_SURROUNDING) {
-            contained = pip_hazard_group(c, s2, qpoi.x, qpoi.y, sub, CG);
+            contained = pip_hazard_group(c, s2, qpoi.x, qpoi.y, sub, n_lanes);
         } else {
             const float4 hp = ldg4(c.haz_poi + s2);
-            contained = pip_query_group(it, m, bb, hp.x, hp.y, sub, CG);
+            contained = pip_query_group(it, m, bb, hp.x, hp.y, sub, n_lanes);
         }
         if (lane == (uint32_t)l && (ldg4(c.haz_poi + s2).w != 0.0f ? contained : !contained)) set_put(L, qs, s2);
     }
@@ -613,69 +612,53 @@ __device__ __forceinline__ void collect_pass(const SetDesc& sd, uint32_t set_ind
     // (cd_engine.rs:276-287), by the query's CG lanes: a candidate without bbox relation
     // collides iff its scope is exterior; the point-in-polygon tests left are split over the
     // CG lanes (containment()'s result).  Only candidates can collide; with more than NC the
-    // virtual root's entries are scanned.
-    if (active && !L.ovf[qs]) {
+    // virtual root's entries are scanned, and in a pass of few queries by the whole wave, one
+    // query after another, as a shallow virtual root has up to every hazard of the layout.  us by
+    // the query's CG lanes / by the wave, items of radius 60 over the 2000-item sheet: 64 queries
+    // 82 / 56, 1000 284 / 95, 10000 333 / 144.
+    uint64_t big = DIRECT ? ballot(active && sub == 0 && !L.ovf[qs] && L.ncand[qs] > NC) : 0ull;
+    for (bool own = true; own || big != 0ull; own = false) {
+        uint32_t q = qs, n_lanes = CG, s0 = sub, base = qs * CG;
+        bool on = active && !L.ovf[qs];
+        if (!own) {
+            q = (uint32_t)__builtin_ctzll(big) / CG;
+            big &= big - 1ull;
+            n_lanes = WAVE;
+            s0 = lane;
+            base = 0u;
+            on = true;
+        }
+        if (!on) continue;
         // the query's transformation, bbox and virtual root entries from LDS, so that no
         // registers hold them over the traversal
-        const Mat m{L.mat[qs][0], L.mat[qs][1], L.mat[qs][2], L.mat[qs][3], L.mat[qs][4], L.mat[qs][5]};
-        const float4 bb = L.qbox[qs];
-        const uint32_t vcnt = L.vcnt[qs], ve0 = L.vbeg[qs];
+        const Mat m{L.mat[q][0], L.mat[q][1], L.mat[q][2], L.mat[q][3], L.mat[q][4], L.mat[q][5]};
+        const float4 bb = L.qbox[q];
+        const uint32_t vcnt = L.vcnt[q], ve0 = L.vbeg[q];
         const float2 qpoi = xform(m, it.poi.x, it.poi.y);
-        const uint32_t nc = L.ncand[qs];
+        const uint32_t nc = L.ncand[q];
         const bool listed = nc <= NC;
-        const uint32_t n_scan = listed ? nc : DIRECT ? 0u : vcnt;
-        for (uint32_t k0 = 0; k0 < n_scan; k0 += CG) {
-            const uint32_t k = k0 + sub;
+        const uint32_t n_scan = listed ? nc : DIRECT && own ? 0u : vcnt;
+        for (uint32_t k0 = 0; k0 < n_scan; k0 += n_lanes) {
+            const uint32_t k = k0 + s0;
             uint32_t sl = 0;
             int rel = REL_DISJOINT;
             bool pend = false;
             if (k < n_scan) {
                 uint32_t sf;
                 if (listed) {
-                    const uint32_t cf = L.cand[qs * NC + k];
+                    const uint32_t cf = L.cand[q * NC + k];
                     sf = (cf & C_SLOT) | ((cf & C_ENTIRE) ? ENTIRE_BIT : 0u);
                 } else {
                     sf = ldg_slot_flags(c.ent + ve0 + k);
                 }
                 sl = sf & SLOT_MASK;
-                if (!(sf & ENTIRE_BIT) && !set_has(L, qs, sl)) {
+                if (!(sf & ENTIRE_BIT) && !set_has(L, q, sl)) {
                     rel = box_almost_relation(ldg4(c.haz_bbox + sl), bb);
                     if (rel == REL_SURROUNDING || rel == REL_ENCLOSED) pend = true;
-                    else if (ldg4(c.haz_poi + sl).w == 0.0f) set_put(L, qs, sl);
+                    else if (ldg4(c.haz_poi + sl).w == 0.0f) set_put(L, q, sl);
                 }
             }
-            containment_group(c, L, it, m, bb, qpoi, qs, sub, lane, pend, sl, rel);
-        }
-    }
-    // few queries in a pass: with more than NC candidates the virtual root's entries are scanned by the
-    // whole wave, as a shallow one has up to every hazard of the layout.  us by the query's CG lanes /
-    // by the wave, items of radius 60 over the 2000-item sheet: 64 queries 82 / 56, 1000 284 / 95,
-    // 10000 333 / 144.  (Not in the plan's passes of CP queries, where it spills 11 more registers.)
-    for (uint32_t q = 0; DIRECT && q < P; q++) {
-        if (L.ncand[q] <= NC || L.ovf[q]) continue;
-        const Mat mq{L.mat[q][0], L.mat[q][1], L.mat[q][2], L.mat[q][3], L.mat[q][4], L.mat[q][5]};
-        const float4 bq = L.qbox[q];
-        const float2 pq = xform(mq, it.poi.x, it.poi.y);
-        const uint32_t n_scan = L.vcnt[q], e0 = L.vbeg[q];
-        for (uint32_t k0 = 0; k0 < n_scan; k0 += WAVE) {
-            const uint32_t k = k0 + lane;
-            const uint32_t sf = k < n_scan ? ldg_slot_flags(c.ent + e0 + k) : ENTIRE_BIT;
-            const uint32_t sl = sf & SLOT_MASK;
-            int rel = REL_DISJOINT;
-            bool pend = false;
-            if (!(sf & ENTIRE_BIT) && !set_has(L, q, sl)) {
-                rel = box_almost_relation(ldg4(c.haz_bbox + sl), bq);
-                if (rel == REL_SURROUNDING || rel == REL_ENCLOSED) pend = true;
-                else if (ldg4(c.haz_poi + sl).w == 0.0f) set_put(L, q, sl);
-            }
-            for (uint64_t pm = __ballot(pend); pm; pm &= pm - 1ull) {
-                const int l = __builtin_ctzll(pm);
-                const uint32_t s2 = (uint32_t)__shfl((int)sl, l, 64);
-                const float4 hp = ldg4(c.haz_poi + s2);
-                const bool contained = __shfl(rel, l, 64) == REL_SURROUNDING ? pip_hazard_wave(c, s2, pq.x, pq.y, lane)
-                                                                             : pip_query_wave(it, mq, bq, hp.x, hp.y, lane);
-                if (lane == (uint32_t)l && (hp.w != 0.0f ? contained : !contained)) set_put(L, q, s2);
-            }
+            containment_group(c, L, it, m, bb, qpoi, q, s0, n_lanes, base, lane, pend, sl, rel);
         }
     }
     wave_sync();
